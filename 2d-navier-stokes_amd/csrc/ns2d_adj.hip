@@ -63,13 +63,14 @@ namespace ns2d {
 
 struct RAdjVariant {
   int NY, TLR, PAIRS, SR;
-  void (*kern)(RAdjArgs);
+  void (*kern[2])(RAdjArgs);   // every column of the read fields; band-limited
 };
 struct KAdjVariant {
   int L, C, T;
   void (*kern)(KAdjArgs);
 };
-#define NS2D_RADJ_ENTRY(NY_, TLR_, PAIRS_, SR_) {NY_, TLR_, PAIRS_, SR_, rpass_adj_kernel<NY_, TLR_, PAIRS_, SR_>},
+#define NS2D_RADJ_ENTRY(NY_, TLR_, PAIRS_, SR_) \
+  {NY_, TLR_, PAIRS_, SR_, {rpass_adj_kernel<NY_, TLR_, PAIRS_, SR_>, rpass_adj_kernel<NY_, TLR_, PAIRS_, SR_, true>}},
 #define NS2D_KADJ_ENTRY(L_, C_, T_) {L_, C_, T_, kpass_adj_kernel<L_, C_, T_>},
 static const RAdjVariant radj_variants[] = {NS2D_RADJ_VARIANTS(NS2D_RADJ_ENTRY)};
 static const KAdjVariant kadj_variants[] = {NS2D_KADJ_VARIANTS(NS2D_KADJ_ENTRY)};
@@ -101,7 +102,7 @@ hipError_t launch_rpass_adj(int nx, int ny, const RAdjArgs& a, hipStream_t s) {
   }
   if (!v) return hipErrorInvalidValue;
   const int units = v->SR ? nx : nx / 2;   // rows or row pairs
-  hipLaunchKernelGGL(v->kern, dim3((units + v->PAIRS - 1) / v->PAIRS), dim3(v->TLR * v->PAIRS), 0, s, a);
+  hipLaunchKernelGGL(v->kern[a.band ? 1 : 0], dim3((units + v->PAIRS - 1) / v->PAIRS), dim3(v->TLR * v->PAIRS), 0, s, a);
   return hipGetLastError();
 }
 

@@ -72,6 +72,15 @@ struct ns2d_handle {
   int cur = 0;             // conj[cur] = ky=0 column of the current stage input
   long iters = 0;
   int hyper_eff = 0;       // HYPER_VISC_FLAG as mutated by the reference (Q3)
+  // Band-limited states.  The 2/3 filter zeroes the right-hand side outside
+  // the disk |k| < kc, so a state that is zero there stays zero there, and the
+  // passes can leave those modes out (kpass_body, rpass_body: BAND).
+  int kc = 0;              // the disk's radius; 0: no such filter, or a forced mode outside it
+  bool band = false;       // w[wcur] is zero outside the disk (found when it is set)
+  bool band_on = false;    // the launches being issued are band-limited
+  bool g_band = false;     // G1..G4 hold the disk's columns alone
+  bool spilled = false;    // w[wcur ^ 1] or the history may hold modes outside the disk
+  unsigned long long epoch = 0;  // of the last state set (marks stat[STAT_SPILL])
   PhysArgs ph{};
   // hipGraph of one period of steps (kernel launches only; see step_impl)
   bool use_graph = true;
@@ -79,7 +88,7 @@ struct ns2d_handle {
   hipGraphExec_t gexec = nullptr;
   struct {
     double dt;
-    int wcur, cur, ring, kvar, rvar, check, period;
+    int wcur, cur, ring, kvar, rvar, check, period, band;
     const double* lam;
   } gkey{};
   // adjoint buffers (allocated on first use)
@@ -100,6 +109,7 @@ struct ns2d_handle {
     int wcur = -1, lc = -1;
     const double* lam = nullptr;
     const double2* tape = nullptr;
+    bool band = false;
   } adj_graph[2];
   // profiling
   bool profiling = false;
@@ -162,8 +172,15 @@ void after_rk_update(ns2d_handle* h) {
   if ((h->p.quirks & NS2D_QUIRK_VISC_ASSIGN) && h->p.drag_flag != 1) h->hyper_eff = 1;
 }
 
+// columns that hold the disk |k| < kc
+int band_columns(const ns2d_handle* h) { return h->kc < h->nyf ? h->kc : h->nyf; }
+// the handle's own launches can leave out the modes outside the disk
+bool band_now(const ns2d_handle* h) { return h->band && kpass_has_band(h->p.nx, h->kvar); }
+
 KPassArgs kbase(ns2d_handle* h) {
   KPassArgs a{};
+  a.band = h->band_on;
+  a.nyc = h->band_on ? band_columns(h) : h->nyf;
   a.w_in = h->w[h->wcur];
   a.w_out = h->w[h->wcur];
   a.acc = h->acc;
@@ -188,32 +205,28 @@ RPassArgs rbase(ns2d_handle* h, int mode) {
   a.tw = h->tw;
   a.ld = h->ld;
   a.nx = h->p.nx;
+  a.band = h->band_on;
+  a.nyc = h->band_on ? band_columns(h) : h->nyf;
   a.mode = mode;
   a.wscale = 1.0 / (double)((long)h->p.nx * h->p.ny);
   return a;
 }
 
 // A [Nx][Ny/2+1] complex array of a caller (host or device memory, `kind`)
-// into / out of the handle's device layout.
-int copy_in(ns2d_handle* h, double2* dst, const void* src, hipMemcpyKind kind) {
+// into / out of the handle's device layout.  kc2 > 0: stat[STAT_SPILL] becomes
+// h->epoch when a mode with |k|^2 >= kc2 is not zero.
+int copy_in(ns2d_handle* h, double2* dst, const void* src, hipMemcpyKind kind, long kc2 = 0) {
   const size_t rowb = h->nyf * sizeof(double2);
-  if constexpr (XT_K == 1) {
-    HIPCHK(hipMemcpy2DAsync(dst, h->ld * sizeof(double2), src, rowb, rowb, h->p.nx, kind, h->stream));
-  } else {
-    HIPCHK(hipMemcpyAsync(h->stage, src, rowb * h->p.nx, kind, h->stream));
-    HIPCHK(launch_relayout(h->stage, dst, h->p.nx, h->nyf, h->ld, 0, h->stream));
-  }
+  HIPCHK(hipMemcpyAsync(h->stage, src, rowb * h->p.nx, kind, h->stream));
+  HIPCHK(launch_relayout(h->stage, dst, h->p.nx, h->nyf, h->ld, 0, kc2, h->stat + STAT_SPILL, h->epoch, h->stream));
   return NS2D_OK;
 }
 
-int copy_out(ns2d_handle* h, void* dst, const double2* src, hipMemcpyKind kind) {
+// kc2 > 0: the modes with |k|^2 >= kc2 are zero and not read
+int copy_out(ns2d_handle* h, void* dst, const double2* src, hipMemcpyKind kind, long kc2 = 0) {
   const size_t rowb = h->nyf * sizeof(double2);
-  if constexpr (XT_K == 1) {
-    HIPCHK(hipMemcpy2DAsync(dst, rowb, src, h->ld * sizeof(double2), rowb, h->p.nx, kind, h->stream));
-  } else {
-    HIPCHK(launch_relayout(src, h->stage, h->p.nx, h->nyf, h->ld, 1, h->stream));
-    HIPCHK(hipMemcpyAsync(dst, h->stage, rowb * h->p.nx, kind, h->stream));
-  }
+  HIPCHK(launch_relayout(src, h->stage, h->p.nx, h->nyf, h->ld, 1, kc2, nullptr, 0, h->stream));
+  HIPCHK(hipMemcpyAsync(dst, h->stage, rowb * h->p.nx, kind, h->stream));
   return NS2D_OK;
 }
 
@@ -239,6 +252,7 @@ void ev_end(ns2d_handle* h) {
 int run_kpass(ns2d_handle* h, const KPassArgs& a) {
   ev_begin(h, KIND_K);
   hipError_t e = launch_kpass(h->p.nx, h->kvar, a, h->stream);
+  if (a.mode & KP_INV) h->g_band = a.band != 0;
   ev_end(h);
   if (e != hipSuccess) return fail(NS2D_ERR_HIP, "kpass launch: %s", hipGetErrorString(e));
   return NS2D_OK;
@@ -254,7 +268,7 @@ int run_rpass(ns2d_handle* h, const RPassArgs& a) {
 
 // G1..G4 (and conj[cur]) from the state: the inverse half of the first RHS
 int prepare_inv(ns2d_handle* h) {
-  if (h->inv_valid) return NS2D_OK;
+  if (h->inv_valid && (h->band_on || !h->g_band)) return NS2D_OK;
   KPassArgs a = kbase(h);
   a.mode = KP_INV;
   a.epi = EPI_FROM_STATE;
@@ -346,7 +360,7 @@ int read_stat(ns2d_handle* h, unsigned long long* st) {
 }
 
 int reset_stat(ns2d_handle* h) {
-  unsigned long long st[STAT_N] = {0ull, 0ull, ~0ull, 0ull};
+  unsigned long long st[STAT_SPILL] = {0ull, 0ull, ~0ull, 0ull, 0ull};
   HIPCHK(hipMemcpyAsync(h->stat, st, sizeof st, hipMemcpyHostToDevice, h->stream));
   HIPCHK(hipStreamSynchronize(h->stream));
   return NS2D_OK;
@@ -354,6 +368,7 @@ int reset_stat(ns2d_handle* h) {
 
 // max|w| of the state into stat[WMAX_CUR] (after clearing it)
 int state_wmax(ns2d_handle* h, double* out, double* wreal) {
+  h->band_on = band_now(h);
   int rc = prepare_inv(h);
   if (rc) return rc;
   const unsigned long long zero = 0ull;
@@ -374,6 +389,7 @@ int state_wmax(ns2d_handle* h, double* out, double* wreal) {
 // GetTimestep's convective rate of the state: the row pass of the state's
 // fields with the CFL reduction (its N output is not used)
 int state_cfl(ns2d_handle* h, double* out) {
+  h->band_on = band_now(h);
   int rc = prepare_inv(h);
   if (rc) return rc;
   const unsigned long long zero = 0ull;
@@ -394,6 +410,7 @@ int state_cfl(ns2d_handle* h, double* out) {
 
 // K = NonlinearRHSBatch(stage input S) into kout, S given by prepared G's
 // and conj[cur]; applies the ForceConjugacy write to the state when enabled.
+// (h->band_on as in the launch that prepared the G's)
 int finish_rhs_into_kout(ns2d_handle* h, bool raw) {
   int rc = run_rpass(h, rbase(h, RP_NL));
   if (rc) return rc;
@@ -545,6 +562,8 @@ static int create_impl(const ns2d_params* p, hipStream_t ext_stream, ns2d_t** ou
   ph.norm2 = std::pow(nf, 2.0);                                              // solver.c:1005
   ph.force_on = p->forcing == NS2D_FORCING_KOLM;
   ph.force_k = p->force_k;
+  if (p->filter == NS2D_FILTER_23 && !(ph.force_on && p->force_k >= p->nx / 3)) h->kc = p->nx / 3;
+  h->band = h->kc > 0;
   ph.force_val = -0.5 * p->force_scale * (double)p->force_k;                 // force.c:537
   if (!(p->quirks & NS2D_QUIRK_KOLM_UNSCALED)) ph.force_val *= (double)((long)p->nx * p->ny);
 
@@ -575,7 +594,7 @@ static int create_impl(const ns2d_params* p, hipStream_t ext_stream, ns2d_t** ou
   }
   if (hipMalloc((void**)&h->pairbuf, sizeof(double2) * 8 * p->nx) != hipSuccess)
     return cleanup(fail(NS2D_ERR_HIP, "hipMalloc failed"));
-  if (XT_K != 1 && hipMalloc((void**)&h->stage, sizeof(double2) * p->nx * h->nyf) != hipSuccess)
+  if (hipMalloc((void**)&h->stage, sizeof(double2) * p->nx * h->nyf) != hipSuccess)
     return cleanup(fail(NS2D_ERR_HIP, "hipMalloc failed"));
   if (hipMalloc((void**)&h->stat, sizeof(unsigned long long) * STAT_N) != hipSuccess)
     return cleanup(fail(NS2D_ERR_HIP, "hipMalloc failed"));
@@ -637,6 +656,8 @@ static int create_impl(const ns2d_params* p, hipStream_t ext_stream, ns2d_t** ou
     }
     h->hyper_eff = p->hyper_flag;
   }
+  if (hipMemsetAsync(h->stat, 0, sizeof(unsigned long long) * STAT_N, h->stream) != hipSuccess)
+    return cleanup(fail(NS2D_ERR_HIP, "memset failed"));
   int rc = reset_stat(h);
   if (rc) return cleanup(rc);
   *out = h;
@@ -677,12 +698,34 @@ int ns2d_destroy(ns2d_t* h) {
   return NS2D_OK;
 }
 
+// A caller's state into w[wcur], and whether it is band-limited (the 2/3
+// filter's disk): one word read back, which waits for the copy.
+static int load_state(ns2d_t* h, const void* src, hipMemcpyKind kind) {
+  h->inv_valid = false;
+  h->band = false;
+  h->epoch += 1;
+  int rc = copy_in(h, h->w[h->wcur], src, kind, (long)h->kc * h->kc);
+  if (rc || h->kc == 0) return rc;
+  unsigned long long spill = 0;
+  HIPCHK(hipMemcpyAsync(&spill, h->stat + STAT_SPILL, sizeof spill, hipMemcpyDeviceToHost, h->stream));
+  HIPCHK(hipStreamSynchronize(h->stream));
+  h->band = spill != h->epoch;
+  if (h->band && h->spilled) {
+    // band-limited launches keep the zeros outside the disk that they find
+    const size_t bytes = h->M * sizeof(double2);
+    HIPCHK(hipMemsetAsync(h->w[h->wcur ^ 1], 0, bytes, h->stream));
+    for (double2* b : h->hist)
+      if (b) HIPCHK(hipMemsetAsync(b, 0, bytes, h->stream));
+    h->spilled = false;
+  }
+  return NS2D_OK;
+}
+
 static int set_state_impl(ns2d_t* h, const void* src, hipMemcpyKind kind) {
   if (!h || !src) return fail(NS2D_ERR_INVALID, "null argument");
   HIPCHK(hipSetDevice(h->p.device));
-  int rc0 = copy_in(h, h->w[h->wcur], src, kind);
+  int rc0 = load_state(h, src, kind);
   if (rc0) return rc0;
-  h->inv_valid = false;
   h->iters = 0;
   h->hyper_eff = h->p.hyper_flag;
   return reset_stat(h);
@@ -691,7 +734,7 @@ static int set_state_impl(ns2d_t* h, const void* src, hipMemcpyKind kind) {
 static int get_state_impl(ns2d_t* h, void* dst, hipMemcpyKind kind) {
   if (!h || !dst) return fail(NS2D_ERR_INVALID, "null argument");
   HIPCHK(hipSetDevice(h->p.device));
-  int rc0 = copy_out(h, dst, h->w[h->wcur], kind);
+  int rc0 = copy_out(h, dst, h->w[h->wcur], kind, h->band ? (long)h->kc * h->kc : 0);
   if (rc0) return rc0;
   HIPCHK(hipStreamSynchronize(h->stream));
   return NS2D_OK;
@@ -724,7 +767,8 @@ static int graph_steps(ns2d_handle* h, double dt, bool check, int period) {
   const int ring = h->p.integrator == NS2D_INT_AB4 ? (int)((h->iters + 1 - 4) % 4) : 0;
   const bool same = h->gexec && h->gkey.dt == dt && h->gkey.wcur == h->wcur && h->gkey.cur == h->cur &&
                     h->gkey.ring == ring && h->gkey.kvar == h->kvar && h->gkey.rvar == h->rvar &&
-                    h->gkey.check == (int)check && h->gkey.period == period && h->gkey.lam == lam;
+                    h->gkey.check == (int)check && h->gkey.period == period && h->gkey.lam == lam &&
+                    h->gkey.band == (int)h->band_on;
   if (!same) {
     drop_graph(h);
     const int cur0 = h->cur, wcur0 = h->wcur, hyp0 = h->hyper_eff;
@@ -754,6 +798,7 @@ static int graph_steps(ns2d_handle* h, double dt, bool check, int period) {
     h->gkey.check = check;
     h->gkey.period = period;
     h->gkey.lam = lam;
+    h->gkey.band = h->band_on;
   }
   HIPCHK(hipGraphLaunch(h->gexec, h->stream));
   h->iters += period;  // cur and wcur are back to their values after a period
@@ -767,6 +812,8 @@ static int step_impl(ns2d_t* h, double dt, long nsteps) {
   HIPCHK(hipSetDevice(h->p.device));
   if (nsteps == 0) return NS2D_OK;
   const bool check = h->p.check_every != 0;
+  h->band_on = band_now(h);
+  if (!h->band_on) h->spilled = true;
   int rc = prepare_inv(h);
   if (rc) return rc;
   const bool ab4 = h->p.integrator == NS2D_INT_AB4;
@@ -819,6 +866,8 @@ int ns2d_rhs(ns2d_t* h, const double* in, double* out) {
   HIPCHK(hipSetDevice(h->p.device));
   int rc = copy_in(h, h->sbuf, in, hipMemcpyHostToDevice);
   if (rc) return rc;
+  h->band_on = false;   // `in` is any field
+  if (h->p.quirks & NS2D_QUIRK_CONJ_GLOBAL) h->band = false;   // and goes into the state's ky = 0 column
   KPassArgs a = kbase(h);
   a.mode = KP_INV;
   a.epi = EPI_FROM_INPUT;
@@ -851,6 +900,7 @@ MeasArgs measures_args(ns2d_handle* h, int with_flux, const double* lam, double*
   a.lam = lam;
   a.quirk_enst_diss = (h->p.quirks & NS2D_QUIRK_ENST_DISS) ? 1 : 0;
   a.nbins = h->nspect;
+  a.klim2 = h->band ? (long)h->kc * h->kc : 0x7fffffffffffffffl;
   a.sbst_lo = 0.0;                   // LWR_SBST_LIM^2, data_types.h:175
   a.sbst_hi = 64.0 * 64.0;           // UPR_SBST_LIM^2, data_types.h:174
   a.ph = h->ph;
@@ -890,6 +940,7 @@ void measures_from_totals(const ns2d_handle* h, const double* tot, double2 wf, i
 // sys_msr.c:125-133: NonlinearRHSBatch(w_hat) (with its ForceConjugacy write
 // into w_hat) into kout; the forcing is subtracted inside the reduction
 int measures_flux_rhs(ns2d_handle* h) {
+  h->band_on = band_now(h);
   int rc = prepare_inv(h);
   if (rc) return rc;
   rc = finish_rhs_into_kout(h, false);
@@ -1019,6 +1070,7 @@ int ns2d_r2c(ns2d_t* h, const double* w, double* w_hat) {
   HIPCHK(hipMemcpyAsync(h->rbuf, w, sizeof(double) * n, hipMemcpyHostToDevice, h->stream));
   hipError_t e = launch_r2c_rows(h->p.nx, h->p.ny, h->rbuf, h->nbuf, h->tw, h->ld, h->stream);
   if (e != hipSuccess) return fail(NS2D_ERR_HIP, "r2c launch: %s", hipGetErrorString(e));
+  h->band_on = false;
   KPassArgs a = kbase(h);
   a.mode = KP_FWD | KP_RAW;
   a.epi = EPI_RHS;
@@ -1037,6 +1089,7 @@ int ns2d_c2r(ns2d_t* h, const double* w_hat, double* w) {
   if (!h->wreal) HIPCHK(hipMalloc((void**)&h->wreal, sizeof(double) * n));
   int rc = copy_in(h, h->sbuf, w_hat, hipMemcpyHostToDevice);
   if (rc) return rc;
+  h->band_on = false;
   KPassArgs a = kbase(h);
   a.mode = KP_INV;
   a.epi = EPI_FROM_INPUT;
@@ -1137,6 +1190,7 @@ struct ns2d_ensemble {
   std::vector<double> dt;
   struct Class {
     int nx = 0, ny = 0, nyf = 0, kvar = 0, rvar = 0;
+    int nyc = 0, band = 0;     // as in every member's arguments
     std::vector<int> idx;
     KPassArgs* dk = nullptr;   // [parity 2][stage 4][members]
     RPassArgs* dr = nullptr;   // [stage 4][members]
@@ -1162,6 +1216,22 @@ void ens_drop(ns2d_ensemble* e) {
   e->gexec = nullptr;
   e->graph = nullptr;
   e->graph_parity = -1;
+}
+
+// A size class is stepped band-limited when every member's state is (and the
+// shapes in use have that form).
+void ens_set_band(ns2d_ensemble* e) {
+  for (auto& c : e->cls) {
+    bool band = kpass_has_band(c.nx, c.kvar);
+    for (int i : c.idx) band = band && band_now(e->m[i]) && band_columns(e->m[i]) == band_columns(e->m[c.idx[0]]);
+    if (c.band != (int)band) e->tables_ok = false;
+    c.band = band;
+    c.nyc = band ? band_columns(e->m[c.idx[0]]) : c.nyf;
+    for (int i : c.idx) {
+      e->m[i]->band_on = band;
+      if (!band) e->m[i]->spilled = true;
+    }
+  }
 }
 
 // (Re)build the per-class argument tables for the members' current buffers.
@@ -1213,10 +1283,11 @@ int ens_launch_step(ns2d_ensemble* e, int p2) {
     hipStream_t cs = fan ? c.stream : e->stream;
     if (fan) HIPCHK(hipStreamWaitEvent(cs, e->fork, 0));
     for (int st = 0; st < 4; ++st) {
-      hipError_t r = launch_rpass_batched(c.nx, c.ny, c.rvar, c.dr + (size_t)st * c.idx.size(), (int)c.idx.size(), cs);
+      hipError_t r = launch_rpass_batched(c.nx, c.ny, c.band, c.rvar, c.dr + (size_t)st * c.idx.size(),
+                                          (int)c.idx.size(), cs);
       if (r != hipSuccess) return fail(NS2D_ERR_HIP, "batched rpass: %s", hipGetErrorString(r));
-      r = launch_kpass_batched(c.nx, c.nyf, c.kvar, c.dk + ((size_t)p2 * 4 + st) * c.idx.size(), (int)c.idx.size(),
-                               cs);
+      r = launch_kpass_batched(c.nx, c.nyc, c.band, c.kvar, c.dk + ((size_t)p2 * 4 + st) * c.idx.size(),
+                               (int)c.idx.size(), cs);
       if (r != hipSuccess) return fail(NS2D_ERR_HIP, "batched kpass: %s", hipGetErrorString(r));
     }
     if (fan) {
@@ -1277,7 +1348,7 @@ int ens_autotune(ns2d_ensemble* e, int reps) {
     int arg = c.rvar;
     for (int v = 0; v < rpass_variant_count(c.ny); ++v) {
       const float ms = step_ms([&](int st) {
-        return launch_rpass_batched(c.nx, c.ny, v, c.dr + (size_t)st * nm, nm, e->stream);
+        return launch_rpass_batched(c.nx, c.ny, c.band, v, c.dr + (size_t)st * nm, nm, e->stream);
       });
       if (ms >= 0.0f && ms < best) {
         best = ms;
@@ -1289,7 +1360,7 @@ int ens_autotune(ns2d_ensemble* e, int reps) {
     arg = c.kvar;
     for (int v = 0; v < kpass_variant_count(c.nx); ++v) {
       const float ms = step_ms([&](int st) {
-        return launch_kpass_batched(c.nx, c.nyf, v, c.dk + (size_t)st * nm, nm, e->stream);
+        return launch_kpass_batched(c.nx, c.nyc, c.band, v, c.dk + (size_t)st * nm, nm, e->stream);
       });
       if (ms >= 0.0f && ms < best) {
         best = ms;
@@ -1361,7 +1432,8 @@ bool jl_field(const std::string& line, const char* key, std::string* out) {
 
 std::string ens_tables_key(const ns2d_ensemble::Class& c) {
   char buf[32];
-  std::snprintf(buf, sizeof buf, "%016llx", shape_table_hash(c.nx, c.ny));
+  // band-limited classes are tuned apart from the others
+  std::snprintf(buf, sizeof buf, "%016llx", shape_table_hash(c.nx, c.ny) ^ (c.band ? 0x9e3779b97f4a7c15ull : 0ull));
   return buf;
 }
 
@@ -1463,7 +1535,7 @@ int ns2d_ens_create(const ns2d_params* members, int n, ns2d_ens_t** out) {
       ns2d_ensemble::Class c;
       c.nx = members[i].nx;
       c.ny = members[i].ny;
-      c.nyf = h->nyf;
+      c.nyf = c.nyc = h->nyf;
       c.kvar = h->kvar;
       c.rvar = h->rvar;
       if (hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking) != hipSuccess ||
@@ -1499,6 +1571,7 @@ int ns2d_ens_step(ns2d_ens_t* e, const double* dt, long nsteps) {
   if (dt_changed) e->tables_ok = false;
   if (nsteps == 0) return NS2D_OK;
   const bool check = e->m[0]->p.check_every != 0;
+  ens_set_band(e);
   for (ns2d_handle* h : e->m) {
     int rc = prepare_inv(h);
     if (rc) return rc;
@@ -1530,6 +1603,12 @@ int ns2d_ens_step(ns2d_ens_t* e, const double* dt, long nsteps) {
       ens_cache_store(e);
     }
     e->tuned = true;
+    // (a class whose tuned shape has no band-limited form turns to all columns)
+    ens_set_band(e);
+    for (ns2d_handle* h : e->m) {
+      int rc = prepare_inv(h);
+      if (rc) return rc;
+    }
   }
   if (s < nsteps) {
     int rc = ens_tables(e, check);
@@ -1563,7 +1642,10 @@ int ns2d_ens_step(ns2d_ens_t* e, const double* dt, long nsteps) {
       s += 1;
     }
   }
-  for (ns2d_handle* h : e->m) h->inv_valid = true;
+  for (ns2d_handle* h : e->m) {
+    h->inv_valid = true;
+    h->g_band = h->band_on;
+  }
   if (check) {
     // SystemCheck of every member's final state (solver.c:2309)
     for (ns2d_handle* h : e->m) {
@@ -1594,6 +1676,7 @@ int ns2d_ens_step(ns2d_ens_t* e, const double* dt, long nsteps) {
 int ns2d_ens_autotune(ns2d_ens_t* e, int reps) {
   if (!e || reps < 1) return fail(NS2D_ERR_INVALID, "bad autotune arguments");
   HIPCHK(hipSetDevice(e->m[0]->p.device));
+  ens_set_band(e);
   for (ns2d_handle* h : e->m) {
     int rc = prepare_inv(h);
     if (rc) return rc;
@@ -1753,6 +1836,8 @@ int vjp_impl(ns2d_handle* h, double dt, long n, long ckpt_every, double2** res) 
   // in the state buffer, so G1..G4 of an earlier state must not be reused.
   // The untaped segments run as ordinary (graph-replayed) steps.
   h->inv_valid = false;
+  h->band_on = band_now(h);
+  if (!h->band_on) h->spilled = true;
   h->iters = 0;
   const int check0 = h->p.check_every;
   h->p.check_every = 0;
@@ -1800,6 +1885,7 @@ int vjp_impl(ns2d_handle* h, double dt, long n, long ckpt_every, double2** res) 
       ka.tw = h->tw;
       ka.nyf = h->nyf;
       ka.ld = h->ld;
+      ka.nyc = h->kc ? band_columns(h) : h->nyf;
       ka.dt = dt;
       ka.ph = h->ph;
       ka.lacc = h->lacc;
@@ -1826,6 +1912,8 @@ int vjp_impl(ns2d_handle* h, double dt, long n, long ckpt_every, double2** res) 
         ra.tw = h->tw;
         ra.nx = h->p.nx;
         ra.ld = h->ld;
+        ra.band = h->band_on;
+        ra.nyc = h->band_on ? band_columns(h) : h->nyf;
         hipError_t e = launch_rpass_adj(h->p.nx, h->p.ny, ra, h->stream);
         if (e != hipSuccess) return fail(NS2D_ERR_HIP, "adjoint rpass: %s", hipGetErrorString(e));
         KAdjArgs kk = ka;
@@ -1883,7 +1971,8 @@ int vjp_impl(ns2d_handle* h, double dt, long n, long ckpt_every, double2** res) 
     const double2* tkey = tape_of(seg);
     ns2d_handle::AdjGraph* g = nullptr;
     for (auto& c : h->adj_graph)
-      if (c.exec && c.dt == dt && c.C == C && c.wcur == h->wcur && c.lc == lc && c.lam == lam1 && c.tape == tkey)
+      if (c.exec && c.dt == dt && c.C == C && c.wcur == h->wcur && c.lc == lc && c.lam == lam1 && c.tape == tkey &&
+          c.band == h->band_on)
         g = &c;
     if (!g) {
       g = !h->adj_graph[0].exec ? &h->adj_graph[0] : !h->adj_graph[1].exec ? &h->adj_graph[1] : &h->adj_graph[seg & 1];
@@ -1908,6 +1997,7 @@ int vjp_impl(ns2d_handle* h, double dt, long n, long ckpt_every, double2** res) 
       g->lc = lc0;
       g->lam = lam1;
       g->tape = tkey;
+      g->band = h->band_on;
       // the capture advanced the host-side parities; the replay does the work
       h->wcur = wcur0;
       lc = lc0;
@@ -1935,7 +2025,7 @@ int ns2d_vjp_device(ns2d_t* h, const void* d_w0, double dt, long nsteps, const v
   HIPCHK(hipSetDevice(h->p.device));
   int rc = adj_alloc(h, 1, 1);
   if (rc) return rc;
-  rc = copy_in(h, h->w[h->wcur], d_w0, hipMemcpyDeviceToDevice);
+  rc = load_state(h, d_w0, hipMemcpyDeviceToDevice);
   if (rc == NS2D_OK) rc = copy_in(h, h->lamp[0], d_lam_T, hipMemcpyDeviceToDevice);
   if (rc) return rc;
   double2* res = nullptr;
@@ -1954,7 +2044,7 @@ int ns2d_vjp(ns2d_t* h, const double* w0, double dt, long nsteps, const double* 
   HIPCHK(hipSetDevice(h->p.device));
   int rc = adj_alloc(h, 1, 1);
   if (rc) return rc;
-  rc = copy_in(h, h->w[h->wcur], w0, hipMemcpyHostToDevice);
+  rc = load_state(h, w0, hipMemcpyHostToDevice);
   if (rc == NS2D_OK) rc = copy_in(h, h->lamp[0], lam_T, hipMemcpyHostToDevice);
   if (rc) return rc;
   double2* res = nullptr;

@@ -78,7 +78,8 @@ enum { EPI_FROM_STATE = 0, EPI_FROM_INPUT = 1, EPI_RHS = 2, EPI_RK1 = 3, EPI_RK2
 enum { RP_NL = 1, RP_W = 2, RP_CFL = 4 };
 
 // device status words (unsigned 64-bit)
-enum { STAT_WMAX_CUR = 0, STAT_WMAX_LAST = 1, STAT_FIRST_BAD = 2, STAT_ITER = 3, STAT_CFL = 4, STAT_N = 5 };
+enum { STAT_WMAX_CUR = 0, STAT_WMAX_LAST = 1, STAT_FIRST_BAD = 2, STAT_ITER = 3, STAT_CFL = 4,
+       STAT_SPILL = 5, STAT_N = 6 };
 
 // per-bin reduction quantities of the measures kernel
 enum {
@@ -122,6 +123,7 @@ struct KPassArgs {
   const double2* tw;
   double2* pairbuf;      // packed (0, Ny/2) column pair: held columns, [split][2][Nx]
   int nyf, ld;
+  int nyc, band;         // columns the pass covers (band: those of the 2/3 disk, else nyf)
   const double* lam;     // per-mode D_fac/dt of the CN update, [Nx][ld]
   int mode, epi;
   // 1: the last column group (one valid column, KS = 1 shapes) runs as two
@@ -139,6 +141,7 @@ struct RPassArgs {
   unsigned long long* wmax;
   const double2* tw;
   int ld, mode;
+  int nyc, band;         // columns read and written (band: those of the 2/3 disk)
   double wscale;
   // RP_CFL: u + iv = (row transform) * cfl_s, grid spacings, result bits
   unsigned long long* cmax;
@@ -159,6 +162,7 @@ struct KAdjArgs {
   const double* lam_prev;  // ... of the previous step (ADJ_S1 with KA_INV)
   const double2* tw;
   int nyf, ld, mode, epi;
+  int nyc;                 // columns the l_n transform is wanted in
   double dt;
   PhysArgs ph;
 };
@@ -169,6 +173,7 @@ struct RAdjArgs {
   double2* bout[4];
   const double2* tw;
   int nx, ld;
+  int nyc, band;           // columns of lin and g (band: those of the 2/3 disk)
 };
 
 struct MeasArgs {
@@ -178,6 +183,7 @@ struct MeasArgs {
   const double* lam;     // per-mode pre_fac (sys_msr.c:160-175), [Nx][ld]
   int nx, ny, ld, quirk_enst_diss;
   int nbins;             // spectrum bins (workgroups past the last one exit)
+  long klim2;            // the state and rhs are zero from this |k|^2 on
   double sbst_lo, sbst_hi;
   PhysArgs ph;
 };
@@ -207,8 +213,11 @@ inline int meas_grid(int nbins) { return (nbins + 8 * MEAS_CHUNK - 1) / (8 * MEA
 hipError_t launch_kpass(int nx, int variant, const KPassArgs& a, hipStream_t s);
 int kpass_variant_count(int nx);
 int kpass_default_variant(int nx, bool ab4);
-hipError_t launch_kpass_batched(int nx, int nyf, int variant, const KPassArgs* tab, int members, hipStream_t s);
-hipError_t launch_rpass_batched(int nx, int ny, int variant, const RPassArgs* tab, int members, hipStream_t s);
+// nyc, band: as in every member's arguments
+hipError_t launch_kpass_batched(int nx, int nyc, int band, int variant, const KPassArgs* tab, int members, hipStream_t s);
+hipError_t launch_rpass_batched(int nx, int ny, int band, int variant, const RPassArgs* tab, int members, hipStream_t s);
+// whether a column-pass shape has a band-limited form (every row-pass shape has)
+bool kpass_has_band(int nx, int variant);
 int kpass_variant_info(int nx, int idx, int* C, int* E, int* T, int* KS);
 hipError_t launch_rpass(int nx, int ny, int variant, const RPassArgs& a, hipStream_t s);
 int rpass_variant_count(int ny);
@@ -219,7 +228,15 @@ unsigned long long shape_table_hash(int nx, int ny);
 hipError_t launch_r2c_rows(int nx, int ny, const double* in, double2* out, const double2* tw, int ld,
                            hipStream_t s);
 hipError_t launch_measures(int nbins, const MeasArgs& a, hipStream_t s);
-hipError_t launch_relayout(const double2* src, double2* dst, int nx, int nyf, int ld, int dir, hipStream_t s);
+// dir 0 (into the device layout), kc2 > 0: *spill = epoch when a mode with
+// |k|^2 >= kc2 is not zero.  dir 1, kc2 > 0: those modes are taken as zero.
+hipError_t launch_relayout(const double2* src, double2* dst, int nx, int nyf, int ld, int dir, long kc2,
+                           unsigned long long* spill, unsigned long long epoch, hipStream_t s);
+hipError_t launch_measures(int nbins, const MeasArgs& a, hipStream_t s);
+// dir 0 (into the device layout) with kc2 > 0: *spill (device) becomes
+// nonzero when a mode with |k|^2 >= kc2 is not zero
+hipError_t launch_relayout(const double2* src, double2* dst, int nx, int nyf, int ld, int dir, long kc2,
+                           unsigned long long* spill, hipStream_t s);
 
 // allocation-free measures: per-device scratch (ns2d_noalloc.hip) sized for
 // the spectrum length of a 4096 x 4096 grid (sys_msr.c:394)

@@ -74,12 +74,12 @@ static const KVariant* find_kvariant(int nx, int idx) {
 }
 
 // Every member of the batch must run a pass with inverse transforms (KS as
-// compiled) and share nyf.
-hipError_t launch_kpass_batched(int nx, int nyf, int variant, const KPassArgs* tab, int members, hipStream_t s) {
+// compiled) and share nyf and nyc.
+hipError_t launch_kpass_batched(int nx, int nyc, int band, int variant, const KPassArgs* tab, int members, hipStream_t s) {
   const KVariant* v = find_kvariant(nx, variant);
-  if (!v) return hipErrorInvalidValue;
-  const int per = v->groups(nyf) * v->KS;
-  hipLaunchKernelGGL(v->batched, dim3(per * members), dim3(v->T), 0, s, tab, per);
+  if (!v || !v->batched[band ? 1 : 0]) return hipErrorInvalidValue;
+  const int per = v->groups(nyc) * v->KS;
+  hipLaunchKernelGGL(v->batched[band ? 1 : 0], dim3(per * members), dim3(v->T), 0, s, tab, per);
   return hipGetLastError();
 }
 
@@ -119,37 +119,27 @@ int kpass_variant_extra(int nx, int idx, int* W, int* PS, int* OFF, int* PK) {
   return 0;
 }
 
+bool kpass_has_band(int nx, int variant) {
+  const KVariant* v = find_kvariant(nx, variant);
+  return v && v->kern[1];
+}
+
 // Launch the kpass for an nx-point column transform.  A pass without inverse
-// transforms (an RHS evaluation) uses a KS = 1 sibling of the same shape:
-// split workgroups exist only to share the inverse fields.
+// transforms (an RHS evaluation) runs one workgroup per column group: split
+// workgroups exist only to share the inverse fields.
 hipError_t launch_kpass(int nx, int variant, const KPassArgs& a, hipStream_t s) {
   const KVariant* v = find_kvariant(nx, variant);
-  if (!v) return hipErrorInvalidValue;
-  if (!(a.mode & KP_INV) && v->KS != 1) {
-    const KVariant* w = nullptr;
-    for (const KVariant& u : kvariant_table())
-      if (u.L == nx && u.KS == 1 && u.C == v->C && u.T == v->T && u.PS == v->PS && u.OFF == v->OFF &&
-          u.PK == v->PK && u.W == v->W && u.PF == v->PF) {
-        w = &u;
-        break;
-      }
-    if (!w)
-      for (const KVariant& u : kvariant_table())
-        if (u.L == nx && u.KS == 1) { w = &u; break; }
-    if (!w) return hipErrorInvalidValue;
-    v = w;
-  }
-  const int groups = v->groups(a.nyf);
+  if (!v || !v->kern[a.band ? 1 : 0]) return hipErrorInvalidValue;
+  const int groups = v->groups(a.nyc);
+  const int splits = (a.mode & KP_INV) ? v->KS : 1;
   // A last column group holding a single column (unpacked, KS = 1, more than
   // one column per group) runs as two half items: it would otherwise be the
   // one workgroup left when every CU has finished its share
   KPassArgs b = a;
-  b.last_split = (v->KS == 1 && v->PK == 0 && v->C > 1 && (a.mode & KP_INV) && a.nyf % v->C == 1) ? 1 : 0;
-  hipLaunchKernelGGL(v->kern, dim3(groups * v->KS + b.last_split), dim3(v->T), 0, s, b);
+  b.last_split = (v->KS == 1 && v->PK == 0 && v->C > 1 && (a.mode & KP_INV) && a.nyc % v->C == 1) ? 1 : 0;
+  hipLaunchKernelGGL(v->kern[a.band ? 1 : 0], dim3(groups * splits + b.last_split), dim3(v->T), 0, s, b);
   return hipGetLastError();
 }
-
-
 
 static const RVariant* find_rvariant(int ny, int idx) {
   int n = 0;
@@ -160,12 +150,12 @@ static const RVariant* find_rvariant(int ny, int idx) {
   return nullptr;
 }
 
-hipError_t launch_rpass_batched(int nx, int ny, int variant, const RPassArgs* tab, int members, hipStream_t s) {
+hipError_t launch_rpass_batched(int nx, int ny, int band, int variant, const RPassArgs* tab, int members, hipStream_t s) {
   const RVariant* v = find_rvariant(ny, variant);
   if (!v) return hipErrorInvalidValue;
   const int units = (v->PFR & 7) >= 2 ? nx : nx / 2;   // rows or row pairs
   const int per = (units + v->PAIRS - 1) / v->PAIRS;
-  hipLaunchKernelGGL(v->batched, dim3(per * members), dim3(v->TLR * v->PAIRS), 0, s, tab, per);
+  hipLaunchKernelGGL(v->batched[band ? 1 : 0], dim3(per * members), dim3(v->TLR * v->PAIRS), 0, s, tab, per);
   return hipGetLastError();
 }
 
@@ -200,7 +190,8 @@ hipError_t launch_rpass(int nx, int ny, int variant, const RPassArgs& a, hipStre
   const RVariant* v = find_rvariant(ny, variant);
   if (!v) return hipErrorInvalidValue;
   const int units = (v->PFR & 7) >= 2 ? nx : nx / 2;   // rows or row pairs
-  hipLaunchKernelGGL((a.mode & RP_CFL) ? v->cfl : v->kern, dim3((units + v->PAIRS - 1) / v->PAIRS),
+  const int b = a.band ? 1 : 0;
+  hipLaunchKernelGGL((a.mode & RP_CFL) ? v->cfl[b] : v->kern[b], dim3((units + v->PAIRS - 1) / v->PAIRS),
                      dim3(v->TLR * v->PAIRS), 0, s, a);
   return hipGetLastError();
 }
@@ -238,18 +229,32 @@ hipError_t launch_r2c_rows(int nx, int ny, const double* in, double2* out, const
 // Between the host layout [Nx][nyf] (contiguous rows, what callers pass) and
 // the device k-space layout (kidx, padding columns ky >= nyf zero): dir 0 packs
 // src (host layout) into dst, dir 1 unpacks src into dst (host layout).
+// kc2 > 0: modes with |k|^2 >= kc2 lie outside the 2/3 filter's disk.  dir 0:
+// *spill = epoch when one of them is not zero (NaN counts as not zero); dir 1:
+// they are zero and not read (NaN once the state has blown up: a NaN in any
+// mode has then reached every mode of the disk, and 0 * NaN is what the
+// filter leaves).
 __global__ __launch_bounds__(256) void relayout_kernel(const double2* __restrict__ src, double2* __restrict__ dst,
-                                                       int nyf, int ld, int nx, int dir) {
+                                                       int nyf, int ld, int nx, int dir, long kc2,
+                                                       unsigned long long* __restrict__ spill,
+                                                       unsigned long long epoch) {
   const int x = blockIdx.y, ky = blockIdx.x * 256 + threadIdx.x;
   if (dir == 0) {
-    if (ky < ld) dst[kidx(x, ky, ld, nx)] = ky < nyf ? src[(size_t)x * nyf + ky] : make_double2(0.0, 0.0);
+    const double2 v = ky < nyf ? src[(size_t)x * nyf + ky] : make_double2(0.0, 0.0);
+    if (ky < ld) dst[kidx(x, ky, ld, nx)] = v;
+    const long kx = kx_of_row(x, nx);
+    if (kc2 > 0 && kx * kx + (long)ky * ky >= kc2 && !(v.x == 0.0 && v.y == 0.0)) *spill = epoch;
   } else if (ky < nyf) {
-    dst[(size_t)x * nyf + ky] = src[kidx(x, ky, ld, nx)];
+    const long kx = kx_of_row(x, nx);
+    const bool out = kc2 > 0 && kx * kx + (long)ky * ky >= kc2;
+    const double2 v = src[out ? kidx(1, 0, ld, nx) : kidx(x, ky, ld, nx)];
+    dst[(size_t)x * nyf + ky] = out ? cscale(0.0, v) : v;
   }
 }
 
-hipError_t launch_relayout(const double2* src, double2* dst, int nx, int nyf, int ld, int dir, hipStream_t s) {
-  hipLaunchKernelGGL(relayout_kernel, dim3((ld + 255) / 256, nx), dim3(256), 0, s, src, dst, nyf, ld, nx, dir);
+hipError_t launch_relayout(const double2* src, double2* dst, int nx, int nyf, int ld, int dir, long kc2,
+                           unsigned long long* spill, unsigned long long epoch, hipStream_t s) {
+  hipLaunchKernelGGL(relayout_kernel, dim3((ld + 255) / 256, nx), dim3(256), 0, s, src, dst, nyf, ld, nx, dir, kc2, spill, epoch);
   return hipGetLastError();
 }
 

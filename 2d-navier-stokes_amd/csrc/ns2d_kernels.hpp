@@ -145,7 +145,19 @@ __device__ __forceinline__ double dealias_factor(const PhysArgs& ph, int kx, int
 // PS: LDS padding (one slot per 2^PS elements); OFF: extra 16-B slots between
 // the slots' lines, which sets where the neighbouring slot's accesses of one
 // wave fall among the LDS banks (adjacent lanes work on adjacent slots)
-template <int L, int C, int T, int KS, int PS, int OFF, int PK, int PF>
+// BAND (2/3 filter, state zero outside the filter's disk |k| < L/3): the
+// right-hand side and so every stage input and later state are zero there
+// too, so the pass runs over the a.nyc columns the disk reaches, reads the
+// state, accumulator, history and coefficients of the disk's rows alone and
+// leaves the others' zeros in memory as they are.
+// On a square grid the disk holds 35 % of the modes and its columns are two
+// thirds of all, so both passes' mixed-space traffic falls to 2/3 and the
+// k-space traffic to a third (RK4CN 816 -> 472 M bytes per step, CN-AB4
+// 264 -> 143 M).  Measured against the passes over all modes, whole solves:
+// 4096^2 CN-AB4 16.28 -> 10.84 ms per 15 steps, 512^2 RK4CN 2.76 -> 2.46 ms
+// per 30, a 24-member ensemble 14.8 -> 12.2 ms per 12; 256^2 and below, where a
+// pass is one chain of latencies, do not change.
+template <int L, int C, int T, int KS, int PS, int OFF, int PK, int PF, bool BAND>
 __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
   constexpr int TL = T / C;        // threads per column
   constexpr int E = L / TL;        // rows per thread
@@ -156,18 +168,33 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
   __shared__ double2 lds[C * LS];
 
   const int tid = threadIdx.x;
+  // a pass without inverse transforms has one work item per column group
+  const bool inv = (a.mode & KP_INV) != 0;
   // with last_split (KS = 1 shapes), work items ngroups-1 and ngroups are the
   // last column group's two halves: two inverse fields each, split 0 writes
-  const int ngroups = ((PK ? a.nyf - 1 : a.nyf) + C - 1) / C;
+  const int ngroups = ((PK ? a.nyf - 1 : a.nyc) + C - 1) / C;
   const bool tail = KS == 1 && a.last_split && wi >= ngroups - 1;
-  const int g = tail ? ngroups - 1 : wi / KS;
-  const int split = tail ? wi - (ngroups - 1) : wi % KS;
+  const int g = tail ? ngroups - 1 : inv ? wi / KS : wi;
+  const int split = tail ? wi - (ngroups - 1) : inv ? wi % KS : 0;
   const int nfs = tail ? 2 : FPS;   // inverse fields of this work item
   const int c = tid % C, l = tid / C;
   const int ky = g * C + c;        // the slot; with PK slot 0 is the (0, Ny/2) pair
   const int nyf = a.nyf, ld = a.ld, nx = L;
   const int H = nyf - 1;           // ky of the Nyquist column
-  const bool colv = ky < (PK ? H : nyf);
+  const bool colv = ky < (PK ? H : a.nyc);
+  // BAND: the disk's radius; row x of column kyv carries a mode inside it
+  constexpr int KC = L / 3;
+  static_assert(!(BAND && PK), "band shapes are unpacked");
+  auto inside = [](int x, int kyv) -> bool {
+    if constexpr (!BAND) return true;
+    const int kx = kx_of_row(x, L);
+    return kx * kx + kyv * kyv < KC * KC;
+  };
+  // BAND: no lane's row of element e lies inside the disk (known at compile time)
+  auto outside_all = [](int e) -> bool { return BAND && TL * e >= KC && TL * e + TL - 1 <= L - KC; };
+  // k-space index of row x; BAND: a row outside the disk takes the row kx =
+  // Nx/2 of its column (its value is then not used)
+  auto kmode = [&](int x, int kyv) -> size_t { return kidx(inside(x, kyv) ? x : L / 2, kyv, ld, nx); };
   const bool pair = PK && ky == 0;
   const bool pblk = PK && g == 0;  // uniform per workgroup
   const bool writer = split == 0;
@@ -214,9 +241,10 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
       const int kyl = colv ? ky : 0;
 #pragma unroll
       for (int it = 0; it < E; ++it) {
+        if (outside_all(it)) continue;
         const int i = l + TL * it;
         const int kx = kx_of_row(i, nx);
-        const size_t idx = kidx(i, kyl, ld, nx);
+        const size_t idx = kmode(i, kyl);
         const bool cj = cf && kx < 0;
         const double2* pw = cj ? a.conj_src + (cj ? -kx : 0) : a.w_in + idx;
         const double2 w = *pw;
@@ -274,7 +302,8 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
     // held live across it
     const int kq = opaque(q ? H : ky);
     const int lq = opaque(l);
-    auto index_of = [&](int it) -> size_t { return kidx(lq + TL * it, kq, ld, nx); };
+    auto index_of = [&](int it) -> size_t { return kmode(lq + TL * it, kq); };
+    auto in_disk = [&](int it) -> bool { return inside(lq + TL * it, kq); };
     if (PKR && q == 1) {
       // S_0 to RH, KH (forward modes) to R
 #pragma unroll
@@ -296,14 +325,15 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
         double2 v = R[e];
         if (a.mode & KP_RAW) {
           // plain unnormalised forward transform (initial conditions)
-        } else if ((kx == 0 && kq == 0) || !colv) {
+        } else if ((kx == 0 && kq == 0) || !colv || !in_disk(e)) {
           // (0,0) = 0; a slot past the last column holds no mode, and its ky
           // may lie past the row's end (ky >= ld), where the per-mode filter
           // table must not be read
           v = make_double2(0.0, 0.0);
         } else {
           v = cscale(nrm, v);                                  // solver.c:1005
-          v = cscale(dealias_factor(ph, kx, kq), v);           // solver.c:1019
+          if constexpr (!BAND) v = cscale(dealias_factor(ph, kx, kq), v);   // solver.c:1019
+          else if (ph.kolm_kill && kx == 0) v = cscale(0.0, v);
           if (ph.force_on && kx == 0 && kq == ph.force_k)      // solver.c:1022-1027
             v.x += ph.force_val;
         }
@@ -318,9 +348,15 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
       const int i = lq + TL * it;
       const int kx = kx_of_row(i, nx);
       const bool cj = conj_fix && kx < 0;
-      const double2* p = cj ? a.conj_src + (cj ? -kx : 0) : a.w_in + kidx(i, kq, ld, nx);
+      const double2* p = cj ? a.conj_src + (cj ? -kx : 0) : a.w_in + kmode(i, kq);
       const double2 v = *p;
       return make_double2(v.x, cj ? -v.y : v.y);
+    };
+    // BAND: rows outside the disk hold zero
+    auto keep = [&](int it, double2 v) -> double2 {
+      if constexpr (!BAND) return v;
+      const bool in = in_disk(it);
+      return make_double2(in ? v.x : 0.0, in ? v.y : 0.0);
     };
     auto acc_at = [&](int it) -> double2 {
       if constexpr (PF != 0) return apre[it];
@@ -334,7 +370,7 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
       case EPI_FROM_STATE:
 #pragma unroll
         for (int it = 0; it < E; ++it) {
-          R[it] = colv ? at(a.w_in, index_of(it)) : make_double2(0.0, 0.0);
+          R[it] = colv ? keep(it, at(a.w_in, index_of(it))) : make_double2(0.0, 0.0);
           if ((it & 3) == 3) asm volatile("" ::: "memory");
         }
         break;
@@ -349,6 +385,7 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
         if (writer && colv) {
 #pragma unroll
           for (int it = 0; it < E; ++it) {
+            if (!in_disk(it)) continue;
             at(a.kout, index_of(it)) = R[it];
             const int kx = kx_of_row(lq + TL * it, nx);
             if (conj_fix && kx < 0) at(a.w_out, index_of(it)) = cconj(at(a.conj_src, -kx));
@@ -359,12 +396,13 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
         if (colv) {
 #pragma unroll
           for (int it = 0; it < E; ++it) {
+            if (outside_all(it)) continue;
             const double2 k = R[it];
-            if (writer) {
+            if (writer && in_disk(it)) {
               at(a.acc, index_of(it)) = cscale(RK4_B1, k);
               if (a.hist_store) at(a.hist_store, index_of(it)) = k;
             }
-            R[it] = cadd(state_at(it), cscale(a.coef, k));     // solver.c:690
+            R[it] = keep(it, cadd(state_at(it), cscale(a.coef, k)));     // solver.c:690
             if ((it & 3) == 3) asm volatile("" ::: "memory");
           }
         }
@@ -375,9 +413,10 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
           const double b = (a.epi == EPI_RK2) ? RK4_B2 : RK4_B3;
 #pragma unroll
           for (int it = 0; it < E; ++it) {
+            if (outside_all(it)) continue;
             const double2 k = R[it];
-            if (writer) at(a.acc, index_of(it)) = cadd(acc_at(it), cscale(b, k));
-            R[it] = cadd(state_at(it), cscale(a.coef, k));     // solver.c:729,768
+            if (writer && in_disk(it)) at(a.acc, index_of(it)) = cadd(acc_at(it), cscale(b, k));
+            R[it] = keep(it, cadd(state_at(it), cscale(a.coef, k)));     // solver.c:729,768
             if ((it & 3) == 3) asm volatile("" ::: "memory");
           }
         }
@@ -386,6 +425,7 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
         if (colv) {
 #pragma unroll
           for (int it = 0; it < E; ++it) {
+            if (outside_all(it)) continue;
             const int kx = kx_of_row(lq + TL * it, nx);
             // every mode computes; the (0,0) mode then takes 0 (solver.c:860)
             const double2 sum = cadd(acc_at(it), cscale(RK4_B4, R[it]));
@@ -393,8 +433,8 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
             const double q = rcp_nr(2.0 + D);
             double2 nw = cadd(cscale((2.0 - D) * q, state_at(it)), cscale(2.0 * a.dt * q, sum));  // :853
             if (kx == 0 && kq == 0) nw = make_double2(0.0, 0.0);
-            if (writer) at(a.w_out, index_of(it)) = nw;
-            R[it] = nw;
+            if (writer && in_disk(it)) at(a.w_out, index_of(it)) = nw;
+            R[it] = keep(it, nw);
             if ((it & 3) == 3) asm volatile("" ::: "memory");
           }
         }
@@ -403,6 +443,7 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
         if (colv) {
 #pragma unroll
           for (int it = 0; it < E; ++it) {
+            if (outside_all(it)) continue;
             const int kx = kx_of_row(lq + TL * it, nx);
             const size_t idx = index_of(it);
             const double2 k = R[it];
@@ -413,11 +454,11 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
             const double q = rcp_nr(2.0 + D);
             double2 nw = cadd(cscale((2.0 - D) * q, state_at(it)), cscale(2.0 * a.dt * q, sum));  // :333
             if (kx == 0 && kq == 0) nw = make_double2(0.0, 0.0);
-            if (writer) {
+            if (writer && in_disk(it)) {
               at(a.h_store, idx) = k;   // newest history entry (solver.c:346-348)
               at(a.w_out, idx) = nw;
             }
-            R[it] = nw;
+            R[it] = keep(it, nw);
             if ((it & 3) == 3) asm volatile("" ::: "memory");
           }
         }
@@ -534,19 +575,19 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
 }
 
 // W: minimum waves per SIMD the register allocation must allow (1 = no limit)
-template <int L, int C, int T, int KS, int PS, int OFF, int PK, int W, int PF>
+template <int L, int C, int T, int KS, int PS, int OFF, int PK, int W, int PF, bool BAND = false>
 __global__ __launch_bounds__(T, W) void kpass_kernel(KPassArgs a) {
-  kpass_body<L, C, T, KS, PS, OFF, PK, PF>(a, xcd_remap((int)blockIdx.x, (int)gridDim.x));
+  kpass_body<L, C, T, KS, PS, OFF, PK, PF, BAND>(a, xcd_remap((int)blockIdx.x, (int)gridDim.x));
 }
 
 // All members of an ensemble size class in one launch: work items
 // [m * per_member, (m+1) * per_member) belong to member m, whose arguments
 // are tab[m] (uniform per workgroup, read with scalar loads).
-template <int L, int C, int T, int KS, int PS, int OFF, int PK, int W, int PF>
+template <int L, int C, int T, int KS, int PS, int OFF, int PK, int W, int PF, bool BAND = false>
 __global__ __launch_bounds__(T, W) void kpass_batched(const KPassArgs* __restrict__ tab, int per_member) {
   const int b = xcd_remap((int)blockIdx.x, (int)gridDim.x);
   const int m = b / per_member;
-  kpass_body<L, C, T, KS, PS, OFF, PK, PF>(tab[m], b - m * per_member);
+  kpass_body<L, C, T, KS, PS, OFF, PK, PF, BAND>(tab[m], b - m * per_member);
 }
 
 // LDS padding of the row passes' line buffers: one 16-B slot per 2^RPS
@@ -579,7 +620,9 @@ constexpr int RPS = NS2D_RPASS_PS;
 // and 2 with the real product's forward transform done at half length
 // (rpass_forward_half).  PFR + 8: the same shape with every twiddle power of
 // its transforms preloaded (TwFull) instead of formed by products.
-template <int NY, int TLR, bool BLOCK, typename TWH>
+// BAND: only the a.nyc columns below the 2/3 filter's radius are read and
+// written (the fields' others are zero, and no column pass reads N there).
+template <int NY, int TLR, bool BLOCK, bool BAND, typename TWH>
 __device__ __forceinline__ void rpass_forward_half(double2 (&w)[NY / TLR], double2* buf, const RPassArgs& a,
                                                    int x0, int l, const TWH& twh);
 
@@ -590,7 +633,7 @@ __device__ __forceinline__ int half_lane(int l) { return (l >> 1) + ((l & 1) ? T
 // tw: the row transforms' twiddle set, twh: the half-length line's.  CFL:
 // the instantiation that can reduce the CFL rate (mode RP_CFL); the step's
 // kernels are built without that code.
-template <int NY, int TLR, int PAIRS, int PFR, bool CFL, typename TW, typename TWH>
+template <int NY, int TLR, int PAIRS, int PFR, bool CFL, bool BAND, typename TW, typename TWH>
 __device__ __forceinline__ void rpass_body_tw(const RPassArgs& a, const int blk, const TW& tw, const TWH& twh) {
   constexpr int T = TLR * PAIRS;
   constexpr int H = NY / 2;
@@ -627,25 +670,29 @@ __device__ __forceinline__ void rpass_body_tw(const RPassArgs& a, const int blk,
       const bool edge = (e == 0 || e == E / 2) && lo == 0;
       const bool mirror = e > E / 2 || (e == E / 2 && lo != 0);
       const int kk = mirror ? NY - ky : ky;
+      // a column past the band takes column 0's address and then zero
+      const bool in = !BAND || kk < a.nyc;
+      const int kl = in ? kk : 0;
       double2 A, B;
       const double fk = (double)kk;
       if (which == 0) {         // u = i ky G1, v = G2
-        const double2 g1 = at(a.g[0], gidx(x, kk, ld));
+        const double2 g1 = at(a.g[0], gidx(x, kl, ld));
         A = make_double2(-fk * g1.y, fk * g1.x);
-        B = at(a.g[1], gidx(x, kk, ld));
+        B = at(a.g[1], gidx(x, kl, ld));
       } else if (which == 1) {  // w_x = G3, w_y = i ky G4
-        A = at(a.g[2], gidx(x, kk, ld));
-        const double2 g4 = at(a.g[3], gidx(x, kk, ld));
+        A = at(a.g[2], gidx(x, kl, ld));
+        const double2 g4 = at(a.g[3], gidx(x, kl, ld));
         B = make_double2(-fk * g4.y, fk * g4.x);
       } else if (which == 2) {  // w of rows x and x+1 = G4
-        A = at(a.g[3], gidx(x, kk, ld));
-        B = at(a.g[3], gidx(x + 1, kk, ld));
+        A = at(a.g[3], gidx(x, kl, ld));
+        B = at(a.g[3], gidx(x + 1, kl, ld));
       } else {                  // w of row x alone
-        A = at(a.g[3], gidx(x, kk, ld));
+        A = at(a.g[3], gidx(x, kl, ld));
         B = make_double2(0.0, 0.0);
       }
       if (edge) { A.y = 0.0; B.y = 0.0; }
       z[e] = mirror ? make_double2(A.x + B.y, B.x - A.y) : make_double2(A.x - B.y, A.y + B.x);
+      if (!in) z[e] = make_double2(0.0, 0.0);
       if ((e & 3) == 3) asm volatile("" ::: "memory");
     }
   };
@@ -677,7 +724,7 @@ __device__ __forceinline__ void rpass_body_tw(const RPassArgs& a, const int blk,
           for (int e = 0; e < E; ++e) {
             const int ky = l + TLR * e;
             const int kk = ky > H ? NY - ky : ky;
-            pre[r][f][e] = at(a.g[f], gidx(x0 + r, kk, ld));
+            pre[r][f][e] = at(a.g[f], gidx(x0 + r, BAND && kk >= a.nyc ? 0 : kk, ld));
           }
       // the same assembly as build() from the loaded values
       auto build_pre = [&](double2* z, int which, const double2 (&g)[4][E]) {
@@ -697,6 +744,7 @@ __device__ __forceinline__ void rpass_body_tw(const RPassArgs& a, const int blk,
           }
           if (kk == 0 || kk == H) { A.y = 0.0; B.y = 0.0; }
           z[e] = mirror ? make_double2(A.x + B.y, B.x - A.y) : make_double2(A.x - B.y, A.y + B.x);
+          if (BAND && kk >= a.nyc) z[e] = make_double2(0.0, 0.0);
         }
       };
 #pragma unroll
@@ -804,13 +852,14 @@ __device__ __forceinline__ void rpass_body_tw(const RPassArgs& a, const int blk,
 
   if (SR && (a.mode & RP_NL) && (BLOCK || valid)) {
     if constexpr (HLF) {
-      rpass_forward_half<NY, TLR, BLOCK>(w, buf, a, x0, l, twh);
+      rpass_forward_half<NY, TLR, BLOCK, BAND>(w, buf, a, x0, l, twh);
     } else {
       fft_reg<NY, TLR, -1, BLOCK, RPS>(w, buf, tw, opaque(l));
       // k = l + TLR*e <= H: every element below E/2, lane 0's element E/2 (k = H)
 #pragma unroll
       for (int e = 0; e <= E / 2; ++e) {
         const int k = l + TLR * e;
+        if (BAND && k >= a.nyc) continue;
         if (e < E / 2) at(a.nout, nidx(x0, k, ld)) = (e == 0 && l == 0) ? make_double2(w[e].x, 0.0) : w[e];
         else if (l == 0) at(a.nout, nidx(x0, k, ld)) = make_double2(w[e].x, 0.0);
       }
@@ -825,7 +874,7 @@ __device__ __forceinline__ void rpass_body_tw(const RPassArgs& a, const int blk,
 #pragma unroll
     for (int e = 0; e <= E / 2; ++e) {
       const int k = l + TLR * e;
-      if (e < E / 2 || l == 0) {
+      if ((e < E / 2 || l == 0) && (!BAND || k < a.nyc)) {
         const double2 p = w[e];
         const double2 qm = cconj(buf[padx_s<RPS>((NY - k) & (NY - 1))]);
         at(a.nout, nidx(x0, k, ld)) = make_double2(0.5 * (p.x + qm.x), 0.5 * (p.y + qm.y));
@@ -835,7 +884,7 @@ __device__ __forceinline__ void rpass_body_tw(const RPassArgs& a, const int blk,
   }
 }
 
-template <int NY, int TLR, int PAIRS, int PFR, bool CFL = false>
+template <int NY, int TLR, int PAIRS, int PFR, bool CFL, bool BAND>
 __device__ __forceinline__ void rpass_body(const RPassArgs& a, const int blk) {
   constexpr int PM = PFR & 7;
   const int l = (int)threadIdx.x % TLR;
@@ -846,17 +895,17 @@ __device__ __forceinline__ void rpass_body(const RPassArgs& a, const int blk) {
     if constexpr (PM >= 4) {
       TwFull<NY / 2, TLR> twh;
       load_twiddles<NY / 2, TLR>(twh, a.tw, half_lane<TLR>(l));
-      rpass_body_tw<NY, TLR, PAIRS, PM, CFL>(a, blk, tw, twh);
+      rpass_body_tw<NY, TLR, PAIRS, PM, CFL, BAND>(a, blk, tw, twh);
     } else {
-      rpass_body_tw<NY, TLR, PAIRS, PM, CFL>(a, blk, tw, a.tw);
+      rpass_body_tw<NY, TLR, PAIRS, PM, CFL, BAND>(a, blk, tw, a.tw);
     }
   } else {
     NS2D_TWIDDLES(NY, TLR, tw, a.tw, l)
     if constexpr (PM >= 4) {
       NS2D_TWIDDLES(NY / 2, TLR, twh, a.tw, half_lane<TLR>(l))
-      rpass_body_tw<NY, TLR, PAIRS, PM, CFL>(a, blk, tw, twh);
+      rpass_body_tw<NY, TLR, PAIRS, PM, CFL, BAND>(a, blk, tw, twh);
     } else {
-      rpass_body_tw<NY, TLR, PAIRS, PM, CFL>(a, blk, tw, a.tw);
+      rpass_body_tw<NY, TLR, PAIRS, PM, CFL, BAND>(a, blk, tw, a.tw);
     }
   }
 }
@@ -883,7 +932,7 @@ __device__ __forceinline__ double swap_lane_pair(double v) {
 // lh = j and j + TLR/2.  The transform leaves Z(lh + TLR*h) in the same
 // distribution; Z(M-k) comes through the line buffer.  Writes N(x0, k) for
 // k = 0..M, each once.
-template <int NY, int TLR, bool BLOCK, typename TWH>
+template <int NY, int TLR, bool BLOCK, bool BAND, typename TWH>
 __device__ __forceinline__ void rpass_forward_half(double2 (&w)[NY / TLR], double2* buf, const RPassArgs& a,
                                                    int x0, int l, const TWH& twh) {
   constexpr int E = NY / TLR, EH = E / 2, M = NY / 2;
@@ -918,8 +967,8 @@ __device__ __forceinline__ void rpass_forward_half(double2 (&w)[NY / TLR], doubl
     if (k == 0) {
       // real-input transform: N(0) and N(M) are real
       at(a.nout, nidx(x0, 0, ld)) = make_double2(Ev.x + Ov.x, 0.0);
-      at(a.nout, nidx(x0, M, ld)) = make_double2(Ev.x - Ov.x, 0.0);
-    } else {
+      if (!BAND || M < a.nyc) at(a.nout, nidx(x0, M, ld)) = make_double2(Ev.x - Ov.x, 0.0);
+    } else if (!BAND || k < a.nyc) {
       at(a.nout, nidx(x0, k, ld)) = cadd(Ev, cmul(pw[h], Ov));
     }
   }
@@ -928,22 +977,22 @@ __device__ __forceinline__ void rpass_forward_half(double2 (&w)[NY / TLR], doubl
 // W: minimum waves per SIMD the register allocation must allow (1 = no limit)
 // Consecutive rows (row pairs) go to one XCD, whose L2 then serves the
 // x-tiles of the mixed-space fields that neighbouring rows share.
-template <int NY, int TLR, int PAIRS, int W, int PFR>
+template <int NY, int TLR, int PAIRS, int W, int PFR, bool BAND = false>
 __global__ __launch_bounds__(TLR * PAIRS, W) void rpass_kernel(RPassArgs a) {
-  rpass_body<NY, TLR, PAIRS, PFR>(a, xcd_remap((int)blockIdx.x, (int)gridDim.x));
+  rpass_body<NY, TLR, PAIRS, PFR, false, BAND>(a, xcd_remap((int)blockIdx.x, (int)gridDim.x));
 }
 
 // the same shape with the CFL-rate reduction compiled in (ns2d_cfl_rate)
-template <int NY, int TLR, int PAIRS, int W, int PFR>
+template <int NY, int TLR, int PAIRS, int W, int PFR, bool BAND = false>
 __global__ __launch_bounds__(TLR * PAIRS, W) void rpass_cfl_kernel(RPassArgs a) {
-  rpass_body<NY, TLR, PAIRS, PFR, true>(a, xcd_remap((int)blockIdx.x, (int)gridDim.x));
+  rpass_body<NY, TLR, PAIRS, PFR, true, BAND>(a, xcd_remap((int)blockIdx.x, (int)gridDim.x));
 }
 
-template <int NY, int TLR, int PAIRS, int W, int PFR>
+template <int NY, int TLR, int PAIRS, int W, int PFR, bool BAND = false>
 __global__ __launch_bounds__(TLR * PAIRS, W) void rpass_batched(const RPassArgs* __restrict__ tab, int per_member) {
   const int b = xcd_remap((int)blockIdx.x, (int)gridDim.x);
   const int m = b / per_member;
-  rpass_body<NY, TLR, PAIRS, PFR>(tab[m], b - m * per_member);
+  rpass_body<NY, TLR, PAIRS, PFR, false, BAND>(tab[m], b - m * per_member);
 }
 
 // ---------------------------------------------------------------------------
@@ -965,7 +1014,10 @@ __global__ __launch_bounds__(TLR * PAIRS, W) void rpass_batched(const RPassArgs*
 // zero imaginary part) instead of a row pair: twice the workgroups, five
 // transforms per workgroup instead of nine.
 // ---------------------------------------------------------------------------
-template <int NY, int TLR, int PAIRS, int SR>
+// BAND: the l_n transform and the G fields reach a.nyc columns (2/3 filter);
+// the products' transforms are wanted in every column (the gradient is not
+// band-limited).
+template <int NY, int TLR, int PAIRS, int SR, bool BAND>
 __device__ __forceinline__ void rpass_adj_body(const RAdjArgs& a, const int blk) {
   constexpr int H = NY / 2;
   constexpr int E = NY / TLR;
@@ -998,11 +1050,14 @@ __device__ __forceinline__ void rpass_adj_body(const RAdjArgs& a, const int blk)
       const bool mirror = e > E / 2 || (e == E / 2 && lo != 0);
       const int kk = mirror ? NY - ky : ky;
       const double fk = (double)kk;
-      double2 A = fa[gidx(xa, kk, ld)], B = hasb ? fb[gidx(xb, kk, ld)] : make_double2(0.0, 0.0);
+      const bool in = !BAND || kk < a.nyc;
+      const int kl = in ? kk : 0;
+      double2 A = fa[gidx(xa, kl, ld)], B = hasb ? fb[gidx(xb, kl, ld)] : make_double2(0.0, 0.0);
       if (mula) A = make_double2(-fk * A.y, fk * A.x);   // times i ky
       if (mulb) B = make_double2(-fk * B.y, fk * B.x);
       if (edge) { A.y = 0.0; B.y = 0.0; }
       z[e] = mirror ? make_double2(A.x + B.y, B.x - A.y) : make_double2(A.x - B.y, A.y + B.x);
+      if (!in) z[e] = make_double2(0.0, 0.0);
       if ((e & 3) == 3) asm volatile("" ::: "memory");
     }
   };
@@ -1059,9 +1114,9 @@ __device__ __forceinline__ void rpass_adj_body(const RAdjArgs& a, const int blk)
   }
 }
 
-template <int NY, int TLR, int PAIRS, int SR>
+template <int NY, int TLR, int PAIRS, int SR, bool BAND = false>
 __global__ __launch_bounds__(TLR * PAIRS) void rpass_adj_kernel(RAdjArgs a) {
-  rpass_adj_body<NY, TLR, PAIRS, SR>(a, xcd_remap((int)blockIdx.x, (int)gridDim.x));
+  rpass_adj_body<NY, TLR, PAIRS, SR, BAND>(a, xcd_remap((int)blockIdx.x, (int)gridDim.x));
 }
 
 template <int L, int C, int T>
@@ -1165,6 +1220,9 @@ __global__ __launch_bounds__(T) void kpass_adj_kernel(KAdjArgs a) {
     if ((e & 3) == 3) asm volatile("" ::: "memory");
   }
   if (!(a.mode & KA_INV)) return;
+  // a column the filter zeroes entirely has a zero l_n transform, which the
+  // band-limited row pass does not read
+  if (ky0 >= a.nyc) return;
 
   // l_n transform of the next stage: x-inverse of Wh .* M .* l_K
   {
@@ -1246,9 +1304,15 @@ __global__ __launch_bounds__(T) void measures_kernel(MeasArgs a) {
   double acc[NQ];
 #pragma unroll
   for (int q = 0; q < NQ; ++q) acc[q] = 0.0;
+  // band-limited state: no mode at or past |k|^2 = klim2 (a bin of such modes
+  // sums zeros: NaN where the state has blown up)
+  if ((long)b * b - b + 1 >= a.klim2) {
+    if (tid < NQ) a.out[(size_t)b * NQ + tid] = 0.0 * a.w_hat[kidx(1, 0, a.ld, nx)].x;
+    return;
+  }
   if (b > 0) {
     // b^2 - b < k^2 <= b^2 + b  <=>  round(|k|) == b
-    const long lo = (long)b * b - b, hi = (long)b * b + b;
+    const long lo = (long)b * b - b, hi = (long)b * b + b < a.klim2 ? (long)b * b + b : a.klim2 - 1;
     const int kxmax = b + 1;
     for (int kxo = tid; kxo <= 2 * kxmax; kxo += T) {
       const int kx = kxo - kxmax;
@@ -1485,10 +1549,10 @@ __global__ __launch_bounds__(T) void measures_kernel(MeasArgs a) {
 
 struct KVariant {
   int L, C, T, KS, PS, OFF, PK, W, PF;
-  void (*kern)(KPassArgs);
-  void (*batched)(const KPassArgs*, int);
-  // work items per column group count: the slots cover nyf columns (PK: nyf-1)
-  int groups(int nyf) const { return ((PK ? nyf - 1 : nyf) + C - 1) / C; }
+  void (*kern[2])(KPassArgs);   // every column; band-limited (unpacked shapes)
+  void (*batched[2])(const KPassArgs*, int);
+  // column groups: the slots cover nyc columns (PK: nyf-1)
+  int groups(int nyc) const { return ((PK ? nyc - 1 : nyc) + C - 1) / C; }
 };
 
 // rpass variants {NY, TLR, PAIRS, W, PFR}: TLR threads per row pair (E = NY/TLR
@@ -1583,9 +1647,9 @@ struct KVariant {
 
 struct RVariant {
   int NY, TLR, PAIRS, W, PFR;
-  void (*kern)(RPassArgs);
-  void (*batched)(const RPassArgs*, int);
-  void (*cfl)(RPassArgs);   // kern with the CFL-rate reduction (mode RP_CFL)
+  void (*kern[2])(RPassArgs);   // every column; band-limited
+  void (*batched[2])(const RPassArgs*, int);
+  void (*cfl[2])(RPassArgs);    // kern with the CFL-rate reduction (mode RP_CFL)
 };
 
 // The shape tables, assembled from the per-length translation units in

@@ -20,8 +20,13 @@ struct KAdd {
 template <int L, int C, int T, int KS, int PS, int OFF, int PK, int W, int PF>
 struct KAdd<true, L, C, T, KS, PS, OFF, PK, W, PF> {
   static void add(std::vector<KVariant>& v) {
-    v.push_back({L, C, T, KS, PS, OFF, PK, W, PF, kpass_kernel<L, C, T, KS, PS, OFF, PK, W, PF>,
-                 kpass_batched<L, C, T, KS, PS, OFF, PK, W, PF>});
+    KVariant k{L, C, T, KS, PS, OFF, PK, W, PF, {kpass_kernel<L, C, T, KS, PS, OFF, PK, W, PF>, nullptr},
+               {kpass_batched<L, C, T, KS, PS, OFF, PK, W, PF>, nullptr}};
+    if constexpr (PK == 0) {
+      k.kern[1] = kpass_kernel<L, C, T, KS, PS, OFF, PK, W, PF, true>;
+      k.batched[1] = kpass_batched<L, C, T, KS, PS, OFF, PK, W, PF, true>;
+    }
+    v.push_back(k);
   }
 };
 
@@ -32,8 +37,10 @@ struct RAdd {
 template <int NY, int TLR, int PAIRS, int W, int PFR>
 struct RAdd<true, NY, TLR, PAIRS, W, PFR> {
   static void add(std::vector<RVariant>& v) {
-    v.push_back({NY, TLR, PAIRS, W, PFR, rpass_kernel<NY, TLR, PAIRS, W, PFR>, rpass_batched<NY, TLR, PAIRS, W, PFR>,
-                 rpass_cfl_kernel<NY, TLR, PAIRS, W, PFR>});
+    v.push_back({NY, TLR, PAIRS, W, PFR,
+                 {rpass_kernel<NY, TLR, PAIRS, W, PFR>, rpass_kernel<NY, TLR, PAIRS, W, PFR, true>},
+                 {rpass_batched<NY, TLR, PAIRS, W, PFR>, rpass_batched<NY, TLR, PAIRS, W, PFR, true>},
+                 {rpass_cfl_kernel<NY, TLR, PAIRS, W, PFR>, rpass_cfl_kernel<NY, TLR, PAIRS, W, PFR, true>}});
   }
 };
 

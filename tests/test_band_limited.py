@@ -1,0 +1,33 @@
+"""The band-limited path (2/3 filter, states zero outside its disk) against the
+path over all modes: on the CPU emulation for every shape of the smallest
+lengths, on the GPU over grids whose Nyquist column lies inside and outside
+the disk, with the shapes' remainders."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+sys.path.insert(0, os.path.join(HERE, "cpuemu"))
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++ with AddressSanitizer")
+def test_band_limited_emulated():
+    import build_emu
+    lib = build_emu.build()
+    env = dict(os.environ, LD_PRELOAD=build_emu.asan_runtime(), NS2D_LIB=lib, NS2D_NO_TORCH="1", NS2D_ENS_CACHE="", NS2D_ENS_TUNE="0",
+               ASAN_OPTIONS="detect_leaks=0")
+    r = subprocess.run([sys.executable, os.path.join(HERE, "cpuemu", "band_cases.py"), "8x16"],
+                       env=env, capture_output=True, text=True, timeout=900)
+    assert r.returncode == 0 and "BAND OK" in r.stdout and "AddressSanitizer" not in r.stderr, \
+        (r.stdout[-2000:], r.stderr[-4000:])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nx,ny", [(8, 8), (64, 64), (32, 256), (256, 64), (128, 128), (256, 256), (512, 512),
+                                   (1024, 256), (256, 1024), (2048, 32), (64, 2048), (4096, 16), (16, 4096)])
+def test_band_limited(nx, ny):
+    import band_cases
+    band_cases.case(nx, ny, True)
