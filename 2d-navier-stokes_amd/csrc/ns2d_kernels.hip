@@ -86,11 +86,18 @@ hipError_t launch_kpass_batched(int nx, int nyc, int band, int variant, const KP
 // Default column-pass shape: index 0 of its length for both integrators (at
 // 4096 the unpacked 1024-thread shape with the 16-slot padding: 320.5
 // against 326.9 us per RK4CN launch for the 512-thread one, 444.2 against
-// 445.0 us for CN-AB4's heavier epilogue, in alternating bench runs).
-int kpass_default_variant(int nx, bool ab4) {
-  (void)nx;
-  (void)ab4;
-  return 0;
+// 445.0 us for CN-AB4's heavier epilogue, in alternating bench runs), but at
+// 128 index 1 from 1024 columns on (128x1024 72.0 against 72.2 us per step,
+// 128x4096 140 against 151; 128x512 47 against 45).
+int kpass_default_variant(int nx, int nyf) {
+  return nx == 128 && nyf > 512 ? 1 : 0;
+}
+
+// Default row-pass shape: index 0 of its length; index 1, row pairs in whole
+// waves, where 2048 rows or more make up for its longer chain (figures at
+// NS2D_RPASS_VARIANTS).
+int rpass_default_variant(int nx, int ny) {
+  return nx >= 2048 && ny >= 32 && ny <= 512 ? 1 : 0;
 }
 
 int kpass_variant_count(int nx) {

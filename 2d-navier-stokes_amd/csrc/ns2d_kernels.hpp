@@ -796,7 +796,7 @@ __device__ __forceinline__ void rpass_body_tw(const RPassArgs& a, const int blk,
     // wave then block max, as for max|w| below (its own LDS words)
     unsigned long long mb = (unsigned long long)__double_as_longlong(cm != cm ? __longlong_as_double(0x7ff8000000000000ll) : cm);
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
+    for (int off = (T < 64 ? T : 64) / 2; off > 0; off >>= 1) {
       const unsigned long long o = __shfl_xor(mb, off, 64);
       mb = o > mb ? o : mb;
     }
@@ -834,7 +834,7 @@ __device__ __forceinline__ void rpass_body_tw(const RPassArgs& a, const int blk,
     // wave then block max; a NaN propagates (its bit pattern compares largest)
     unsigned long long mb = (unsigned long long)__double_as_longlong(m);
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
+    for (int off = (T < 64 ? T : 64) / 2; off > 0; off >>= 1) {
       const unsigned long long o = __shfl_xor(mb, off, 64);
       mb = o > mb ? o : mb;
     }
@@ -1419,16 +1419,26 @@ __global__ __launch_bounds__(T) void measures_kernel(MeasArgs a) {
 // 1024 one column per 256 threads, 2 splits, 16-slot padding (-7.5 %, and
 // -0.3 % per step against 8-slot padding in interleaved timing); 512 one column per
 // 128 threads, 4 splits (-5 %); 256 one column per wave, 4 splits (-38 %,
-// no workgroup barriers).
+// no workgroup barriers).  Below 256 a launch is one chain of latencies: two
+// points per lane and the four fields on four workgroups give the shortest
+// (64x64 114 -> 62 us per step against 16 columns per wave and workgroup, 128x512
+// 104 -> 45); four points per lane once a launch has thousands of columns
+// (128x4096 140 against 151 us).
 #define NS2D_KPASS_VARIANTS(X) \
+  X(8, 16, 64, 4, 3, 1, 0, 1, 0) \
   X(8, 16, 64, 1, 3, 1, 0, 1, 0) \
   X(8, 16, 64, 1, 3, 1, 1, 1, 0) \
+  X(16, 8, 64, 4, 3, 1, 0, 1, 0) \
   X(16, 16, 64, 1, 3, 1, 0, 1, 0) \
   X(16, 16, 64, 1, 3, 1, 1, 1, 0) \
+  X(32, 4, 64, 4, 3, 1, 0, 1, 0) \
   X(32, 16, 64, 1, 3, 1, 0, 1, 0) \
   X(32, 16, 64, 1, 3, 1, 1, 1, 0) \
+  X(64, 2, 64, 4, 3, 1, 0, 1, 0) \
   X(64, 16, 64, 1, 3, 1, 0, 1, 0) \
   X(64, 16, 64, 1, 3, 1, 1, 1, 0) \
+  X(128, 1, 64, 4, 3, 1, 0, 1, 0) \
+  X(128, 2, 64, 4, 3, 1, 0, 1, 0) \
   X(128, 16, 128, 1, 3, 1, 0, 1, 0) \
   X(128, 16, 128, 1, 3, 1, 1, 1, 0) \
   X(128, 8, 64, 2, 3, 1, 1, 1, 0) \
@@ -1576,36 +1586,50 @@ struct KVariant {
 // twiddle power preloaded, one-wave rows only): 256, 48.84 against 51.06 for
 // the same shape forming the powers, so the 256 default; 512 and 1024 slower
 // (89.4 against 88.3, 185.2 against 164.7: a likely reason, not measured,
-// is the scattered table reads of every wave at the kernel's start).
+// is the scattered table reads of every wave at the kernel's start).  Below
+// 256 one row per workgroup with two to four points per lane, all loads up
+// front, is the shortest chain (64x64 62 -> 36 us per step against 16-row-pair
+// waves, 32x32 59 -> 34, 128x128 65 -> 38); with 2048 rows and more the pass is
+// bound by its traffic and whole waves of row pairs win (4096x64 212 against
+// 254, 4096x256 261 against 283, 4096x512 294 against 305): index 1 of each
+// length (rpass_default_variant).  256 with the fields loaded up front as well:
+// 46.7 against 47.8.
 #define NS2D_RPASS_VARIANTS(X) \
+  X(8, 4, 1, 1, 3) \
   X(8, 1, 64, 1, 0) \
+  X(16, 8, 1, 1, 3) \
   X(16, 1, 64, 1, 0) \
   X(16, 4, 1, 1, 4) \
   X(16, 4, 1, 1, 10) \
   X(16, 4, 1, 1, 12) \
-  X(32, 2, 32, 1, 0) \
+  X(32, 16, 1, 1, 3) \
   X(32, 4, 16, 1, 0) \
-  X(64, 4, 16, 1, 0) \
+  X(32, 2, 32, 1, 0) \
+  X(64, 16, 1, 1, 3) \
   X(64, 8, 8, 1, 0) \
-  X(128, 8, 8, 1, 0) \
+  X(64, 4, 16, 1, 0) \
+  X(128, 64, 1, 1, 11) \
   X(128, 16, 4, 1, 0) \
+  X(128, 8, 8, 1, 0) \
   X(128, 32, 2, 1, 0) \
+  X(256, 64, 1, 1, 11) \
+  X(256, 32, 2, 1, 0) \
   X(256, 64, 1, 1, 10) \
   X(256, 64, 1, 1, 2) \
   X(256, 64, 1, 1, 0) \
   X(256, 64, 1, 1, 1) \
   X(256, 16, 4, 1, 0) \
-  X(256, 32, 2, 1, 0) \
   X(256, 64, 1, 1, 3) \
   X(256, 64, 1, 1, 4) \
   X(512, 64, 1, 1, 4) \
+  X(512, 64, 4, 1, 0) \
   X(512, 64, 1, 1, 0) \
   X(512, 64, 1, 1, 2) \
   X(512, 32, 2, 1, 0) \
   X(512, 128, 1, 1, 0) \
   X(512, 128, 1, 1, 1) \
   X(512, 64, 2, 1, 0) \
-  X(512, 64, 4, 1, 0) \
+  X(512, 64, 1, 1, 11) \
   X(512, 128, 1, 1, 2) \
   X(512, 64, 1, 1, 3) \
   X(1024, 64, 1, 1, 3) \

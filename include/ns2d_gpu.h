@@ -202,8 +202,8 @@ int ns2d_variant_info(int pass, int n, int idx, int* shape4);
  * table instead of forming them by products (row pass only; bit 1 then means
  * its G fields are loaded up front). */
 int ns2d_variant_extra(int pass, int n, int idx, int* extra4);
-/* The shape a new handle with this integrator (NS2D_INT_*) runs for a
- * transform length n unless NS2D_KPASS_VARIANT_<Nx> / NS2D_RPASS_VARIANT_<Ny>
+/* The shape a new handle with this integrator (NS2D_INT_*) runs on a square
+ * grid of length n (other grids may start from a neighbouring index) unless NS2D_KPASS_VARIANT_<Nx> / NS2D_RPASS_VARIANT_<Ny>
  * name another.  Needs no GPU. */
 int ns2d_default_variant(int pass, int n, int integrator, int* idx);
 int ns2d_set_variant(ns2d_t* h, int pass, int idx);
