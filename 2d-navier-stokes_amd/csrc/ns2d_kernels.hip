@@ -93,11 +93,14 @@ int kpass_default_variant(int nx, int nyf) {
   return nx == 128 && nyf > 512 ? 1 : 0;
 }
 
-// Default row-pass shape: index 0 of its length; index 1, row pairs in whole
-// waves, where 2048 rows or more make up for its longer chain (figures at
-// NS2D_RPASS_VARIANTS).
+// Default row-pass shape.  Up to 512 points the first two shapes of a length
+// are row pairs in whole waves and single rows: single rows for their shorter
+// chain, row pairs from 2048 rows on, where the pass is bound by its traffic
+// (figures at NS2D_RPASS_VARIANTS).
 int rpass_default_variant(int nx, int ny) {
-  return nx >= 2048 && ny >= 32 && ny <= 512 ? 1 : 0;
+  const bool tall = nx >= 2048;
+  if (ny < 256) return tall ? 0 : 1;   // index 0: row pairs
+  return tall && ny <= 512 ? 1 : 0;    // index 1: row pairs
 }
 
 int kpass_variant_count(int nx) {

@@ -1591,25 +1591,25 @@ struct KVariant {
 // front, is the shortest chain (64x64 62 -> 36 us per step against 16-row-pair
 // waves, 32x32 59 -> 34, 128x128 65 -> 38); with 2048 rows and more the pass is
 // bound by its traffic and whole waves of row pairs win (4096x64 212 against
-// 254, 4096x256 261 against 283, 4096x512 294 against 305): index 1 of each
-// length (rpass_default_variant).  256 with the fields loaded up front as well:
+// 254, 4096x256 261 against 283, 4096x512 294 against 305): indices 0 and 1 of
+// these lengths, chosen by rpass_default_variant.  256 with the fields loaded up front as well:
 // 46.7 against 47.8.
 #define NS2D_RPASS_VARIANTS(X) \
-  X(8, 4, 1, 1, 3) \
   X(8, 1, 64, 1, 0) \
-  X(16, 8, 1, 1, 3) \
+  X(8, 4, 1, 1, 3) \
   X(16, 1, 64, 1, 0) \
+  X(16, 8, 1, 1, 3) \
   X(16, 4, 1, 1, 4) \
   X(16, 4, 1, 1, 10) \
   X(16, 4, 1, 1, 12) \
-  X(32, 16, 1, 1, 3) \
   X(32, 4, 16, 1, 0) \
+  X(32, 16, 1, 1, 3) \
   X(32, 2, 32, 1, 0) \
-  X(64, 16, 1, 1, 3) \
   X(64, 8, 8, 1, 0) \
+  X(64, 16, 1, 1, 3) \
   X(64, 4, 16, 1, 0) \
-  X(128, 64, 1, 1, 11) \
   X(128, 16, 4, 1, 0) \
+  X(128, 64, 1, 1, 11) \
   X(128, 8, 8, 1, 0) \
   X(128, 32, 2, 1, 0) \
   X(256, 64, 1, 1, 11) \
