@@ -628,8 +628,8 @@ static int create_impl(const ns2d_params* p, hipStream_t ext_stream, ns2d_t** ou
   if (const char* g = std::getenv("NS2D_GRAPH")) h->use_graph = std::atoi(g) != 0;
   // pass shapes: built-in defaults, or NS2D_KPASS_VARIANT_<Nx> / NS2D_RPASS_VARIANT_<Ny>
   {
-    h->kvar = kpass_default_variant(p->nx, h->nyf);
-    h->rvar = rpass_default_variant(p->nx, p->ny);
+    h->kvar = kpass_default_variant(p->nx, h->kc ? band_columns(h) : h->nyf);
+    h->rvar = rpass_default_variant(p->nx, p->ny, p->integrator == NS2D_INT_AB4);
     char name[64];
     std::snprintf(name, sizeof name, "NS2D_KPASS_VARIANT_%d", p->nx);
     const char* env = std::getenv(name);

@@ -267,7 +267,11 @@ __device__ __forceinline__ void apply_butterfly_twiddles(double2* x, const TwFul
   }
 }
 
-template <int N, int TL, int SIGN, bool BLOCK, int P, int PS, int OFF, typename TW>
+// SPL: the exchange passes the real and then the imaginary parts through a
+// line buffer of N doubles (padded like the complex one), for shapes whose
+// workgroups per CU are limited by LDS: half the buffer, two barriers more per
+// exchange.
+template <int N, int TL, int SIGN, bool BLOCK, int P, int PS, int OFF, bool SPL, typename TW>
 __device__ __forceinline__ void fft_reg_pass(double2* v, double2* buf, const TW& tw, int l) {
   constexpr int E = N / TL;
   constexpr int REM = N / P;
@@ -289,6 +293,14 @@ __device__ __forceinline__ void fft_reg_pass(double2* v, double2* buf, const TW&
       if constexpr (LAST) {
 #pragma unroll
         for (int r = 0; r < R; ++r) v[m + r * NB] = x[r];
+      } else if constexpr (SPL) {
+        double* const rb = reinterpret_cast<double*>(buf);
+        const int j0 = (i - k) * R + k;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          rb[padx_s<PS>(j0 + r * P)] = x[r].x;
+          v[m + r * NB].y = x[r].y;   // written after the real parts have been read
+        }
       } else {
         const int j0 = (i - k) * R + k;
 #pragma unroll
@@ -297,11 +309,29 @@ __device__ __forceinline__ void fft_reg_pass(double2* v, double2* buf, const TW&
     }
     if constexpr (!LAST) {
       xsync<BLOCK>();
+      if constexpr (SPL) {
+        double* const rb = reinterpret_cast<double*>(buf);
 #pragma unroll
-      for (int e = 0; e < E; ++e) v[e] = buf[fft_slot<PS, P, R>(l + TL * e)];
+        for (int e = 0; e < E; ++e) v[e].x = rb[padx_s<PS>(l + TL * e)];
+        xsync<BLOCK>();
+#pragma unroll
+        for (int m = 0; m < NB; ++m) {
+          const int i = l + TL * m;
+          const int k = i & (P - 1);
+          const int j0 = (i - k) * R + k;
+#pragma unroll
+          for (int r = 0; r < R; ++r) rb[padx_s<PS>(j0 + r * P)] = v[m + r * NB].y;
+        }
+        xsync<BLOCK>();
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e].y = rb[padx_s<PS>(l + TL * e)];
+      } else {
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e] = buf[fft_slot<PS, P, R>(l + TL * e)];
+      }
       xsync<BLOCK>();
       fft_reg_pass<N, TL, SIGN, BLOCK, P * R, PS,
-                   OFF + (P > 1 ? NB * TwSlots<TW>::template per_butterfly<R>() : 0)>(v, buf, tw, l);
+                   OFF + (P > 1 ? NB * TwSlots<TW>::template per_butterfly<R>() : 0), SPL>(v, buf, tw, l);
     }
   }
 }
@@ -311,12 +341,12 @@ __device__ __forceinline__ void fft_reg_pass(double2* v, double2* buf, const TW&
 // All TL threads of the line (and, with BLOCK, every thread of the block)
 // must call.
 // tw: the global table (const double2*) or the thread's preloaded TwReg<N, TL>
-// (loaded with the same l).
-template <int N, int TL, int SIGN, bool BLOCK, int PS = 3, typename TW>
+// (loaded with the same l).  SPL: buf holds padx_s<PS>(N) doubles.
+template <int N, int TL, int SIGN, bool BLOCK, int PS = 3, bool SPL = false, typename TW>
 __device__ __forceinline__ void fft_reg(double2* v, double2* buf, const TW& tw, int l) {
   static_assert((N & (N - 1)) == 0 && N >= 2 && N % TL == 0, "bad FFT shape");
   static_assert(N <= NS2D_TW_LEN, "twiddle table too short");
-  fft_reg_pass<N, TL, SIGN, BLOCK, 1, PS, 0>(v, buf, tw, l);
+  fft_reg_pass<N, TL, SIGN, BLOCK, 1, PS, 0, SPL>(v, buf, tw, l);
 }
 
 }  // namespace ns2d

@@ -212,8 +212,8 @@ inline int meas_grid(int nbins) { return (nbins + 8 * MEAS_CHUNK - 1) / (8 * MEA
 
 hipError_t launch_kpass(int nx, int variant, const KPassArgs& a, hipStream_t s);
 int kpass_variant_count(int nx);
-int kpass_default_variant(int nx, int nyf);
-int rpass_default_variant(int nx, int ny);
+int kpass_default_variant(int nx, int nyc);
+int rpass_default_variant(int nx, int ny, bool ab4);
 // nyc, band: as in every member's arguments
 hipError_t launch_kpass_batched(int nx, int nyc, int band, int variant, const KPassArgs* tab, int members, hipStream_t s);
 hipError_t launch_rpass_batched(int nx, int ny, int band, int variant, const RPassArgs* tab, int members, hipStream_t s);

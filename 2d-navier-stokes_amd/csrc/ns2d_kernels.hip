@@ -83,24 +83,69 @@ hipError_t launch_kpass_batched(int nx, int nyc, int band, int variant, const KP
   return hipGetLastError();
 }
 
-// Default column-pass shape: index 0 of its length for both integrators (at
-// 4096 the unpacked 1024-thread shape with the 16-slot padding: 320.5
-// against 326.9 us per RK4CN launch for the 512-thread one, 444.2 against
-// 445.0 us for CN-AB4's heavier epilogue, in alternating bench runs), but at
-// 128 index 1 from 1024 columns on (128x1024 72.0 against 72.2 us per step,
-// 128x4096 140 against 151; 128x512 47 against 45).
-int kpass_default_variant(int nx, int nyf) {
-  return nx == 128 && nyf > 512 ? 1 : 0;
+static int k_index(int L, int C, int T, int KS, int PS, int OFF, int PF) {
+  int n = 0;
+  for (const KVariant& v : kvariant_table()) {
+    if (v.L != L) continue;
+    if (v.C == C && v.T == T && v.KS == KS && v.PS == PS && v.OFF == OFF && v.PF == PF && v.PK == 0 && v.W == 1) return n;
+    ++n;
+  }
+  return 0;
 }
 
-// Default row-pass shape.  Up to 512 points the first two shapes of a length
-// are row pairs in whole waves and single rows: single rows for their shorter
-// chain, row pairs from 2048 rows on, where the pass is bound by its traffic
-// (figures at NS2D_RPASS_VARIANTS).
-int rpass_default_variant(int nx, int ny) {
+static int r_index(int NY, int TLR, int PAIRS, int PFR) {
+  int n = 0;
+  for (const RVariant& v : rvariant_table()) {
+    if (v.NY != NY) continue;
+    if (v.TLR == TLR && v.PAIRS == PAIRS && v.PFR == PFR) return n;
+    ++n;
+  }
+  return 0;
+}
+
+// Default column-pass shape for passes over nyc columns: index 0 of its length
+// (at 4096 the unpacked 1024-thread shape with the 16-slot padding: 320.5
+// against 326.9 us per RK4CN launch for the 512-thread one, 444.2 against
+// 445.0 us for CN-AB4's heavier epilogue, in alternating bench runs) where
+// the columns roughly fill the CUs once; with many more columns, shapes that
+// redo less of the forward transform, with fewer, shapes of one column per
+// workgroup.  Column pass, us per launch, against index 0:
+//   128   > 512 columns   2 columns, 4 points per lane  (128x4096 RK4CN step 140 / 151)
+//   256   > 1024          2 splits instead of 4         2049 columns 21.7 / 26.5
+//   512   > 400           2 columns, 2 splits           513: 21.2 / 22.0, 2049: 37.5 / 53.2
+//   1024  > 700           2 columns of 512 threads      1025: 41.7 / 45.6, 2049: 76.7 / 97.3
+//   2048  <= 300          1 column, 2 splits            257: 27.5 / 34.0
+//   2048  <= 700          1 column                      513: 40.8 / 46.0, 683: 45.7 / 46.7
+//   4096  301 .. 700      1 column, exchanges of doubles 513: 96.2 / 104.3 (257: 54.8 / 49.9)
+int kpass_default_variant(int nx, int nyc) {
+  if (nx == 128 && nyc > 512) return k_index(128, 2, 64, 4, 3, 1, 0);
+  if (nx == 256 && nyc > 1024) return k_index(256, 1, 64, 2, 3, 1, 0);
+  if (nx == 512 && nyc > 400) return k_index(512, 2, 256, 2, 4, 8, 0);
+  if (nx == 1024 && nyc > 700) return k_index(1024, 2, 512, 2, 4, 8, 0);
+  if (nx == 2048 && nyc <= 300) return k_index(2048, 1, 256, 2, 3, 1, 0);
+  if (nx == 2048 && nyc <= 700) return k_index(2048, 1, 256, 1, 3, 1, 0);
+  if (nx == 4096 && nyc > 300 && nyc <= 700) return k_index(4096, 1, 512, 1, 3, 1, 2);
+  return 0;
+}
+
+// Default row-pass shape: index 0 of its length, but
+//   up to 128   single rows (index 0 is row pairs in whole waves) for their
+//               shorter chain, below 2048 rows
+//   256, 512    row pairs in whole waves from 2048 rows on, where the pass is
+//               bound by its traffic (figures at NS2D_RPASS_VARIANTS)
+//   1024        from 2048 rows on, the fields loaded as needed: two waves per
+//               SIMD instead of one (2048 rows 27.6 / 30.2 us per launch, 4096
+//               rows 44.4 / 51.5)
+//   4096        up to 512 rows the 512-thread shape (512 rows 22.6 / 23.3);
+//               with CN-AB4's max|w| in every step the fields loaded as needed
+int rpass_default_variant(int nx, int ny, bool ab4) {
   const bool tall = nx >= 2048;
   if (ny < 256) return tall ? 0 : 1;   // index 0: row pairs
-  return tall && ny <= 512 ? 1 : 0;    // index 1: row pairs
+  if (ny <= 512) return tall ? 1 : 0;  // index 1: row pairs
+  if (ny == 1024 && tall) return r_index(1024, 64, 1, 2);
+  if (ny == 4096 && nx <= 512) return r_index(4096, 512, 1, 2);
+  if (ny == 4096 && ab4) return r_index(4096, 256, 1, 18);
+  return 0;
 }
 
 int kpass_variant_count(int nx) {
@@ -125,7 +170,7 @@ int kpass_variant_extra(int nx, int idx, int* W, int* PS, int* OFF, int* PK) {
   *W = v->W;
   *PS = v->PS;
   *OFF = v->OFF;
-  *PK = (v->PK != 0) | (v->PF << 1) | ((v->PK == 2) << 2);
+  *PK = (v->PK != 0) | ((v->PF & 1) << 1) | ((v->PK == 2) << 2) | (((v->PF & 2) != 0) << 6);
   return 0;
 }
 
@@ -192,7 +237,8 @@ int rpass_variant_extra(int ny, int idx, int* W, int* PS, int* OFF, int* PK) {
   *PS = 3;
   *OFF = 1;
   const int pm = v->PFR & 7;
-  *PK = ((pm == 1 || pm == 3 || pm == 4) << 1) | ((pm >= 2) << 3) | ((pm >= 4) << 4) | (((v->PFR & 8) != 0) << 5);
+  *PK = ((pm == 1 || pm == 3 || pm == 4) << 1) | ((pm >= 2) << 3) | ((pm >= 4) << 4) | (((v->PFR & 8) != 0) << 5) |
+        (((v->PFR & 16) != 0) << 6);
   return 0;
 }
 

@@ -157,15 +157,18 @@ __device__ __forceinline__ double dealias_factor(const PhysArgs& ph, int kx, int
 // 4096^2 CN-AB4 16.28 -> 10.84 ms per 15 steps, 512^2 RK4CN 2.76 -> 2.46 ms
 // per 30, a 24-member ensemble 14.8 -> 12.2 ms per 12; 256^2 and below, where a
 // pass is one chain of latencies, do not change.
-template <int L, int C, int T, int KS, int PS, int OFF, int PK, int PF, bool BAND>
+template <int L, int C, int T, int KS, int PS, int OFF, int PK, int PFX, bool BAND>
 __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
+  constexpr int PF = PFX & 1;
+  constexpr bool SPL = (PFX & 2) != 0;   // exchanges of doubles (fft_reg)
+  static_assert(!(SPL && PK), "the packed pair needs a complex line buffer");
   constexpr int TL = T / C;        // threads per column
   constexpr int E = L / TL;        // rows per thread
   constexpr int LS = padx_s<PS>(L) + OFF;
   constexpr int FPS = 4 / KS;      // inverse fields per split
   constexpr bool BLOCK = T > 64;
   static_assert(T % C == 0 && L % TL == 0 && E >= 2 && 4 % KS == 0, "bad kpass shape");
-  __shared__ double2 lds[C * LS];
+  __shared__ double lds[C * LS * (SPL ? 1 : 2)] __attribute__((aligned(16)));
 
   const int tid = threadIdx.x;
   // a pass without inverse transforms has one work item per column group
@@ -199,7 +202,7 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
   const bool pblk = PK && g == 0;  // uniform per workgroup
   const bool writer = split == 0;
   const PhysArgs& ph = a.ph;
-  double2* buf = lds + c * LS;
+  double2* buf = reinterpret_cast<double2*>(lds + c * LS * (SPL ? 1 : 2));
   NS2D_TWIDDLES(L, TL, tw, a.tw, l)
   // the pair's held columns (see above)
   double2* __restrict__ hold = a.pairbuf + (size_t)split * 2 * L;
@@ -270,7 +273,7 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
       else R[e] = colv ? at(a.nin, nidx(x, ky, ld)) : make_double2(0.0, 0.0);
       if ((e & 3) == 3) asm volatile("" ::: "memory");
     }
-    fft_reg<L, TL, -1, BLOCK, PS>(R, buf, tw, opaque(l));
+    fft_reg<L, TL, -1, BLOCK, PS, SPL>(R, buf, tw, opaque(l));
     if (pblk) {
       if (pair) {
 #pragma unroll
@@ -548,7 +551,7 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
 #pragma unroll
       for (int e = 0; e < E; ++e) F[e] = derive(f, R[e], kx_of_row(l_o + TL * e, nx), ky_o);
     }
-    fft_reg<L, TL, +1, BLOCK, PS>(F, buf, tw, l_o);
+    fft_reg<L, TL, +1, BLOCK, PS, SPL>(F, buf, tw, l_o);
     double2* __restrict__ gout = a.g[f];
     if (pair) {
       double* __restrict__ g4 = reinterpret_cast<double*>(a.g[3]);
@@ -595,6 +598,9 @@ __global__ __launch_bounds__(T, W) void kpass_batched(const KPassArgs* __restric
 #define NS2D_RPASS_PS 3
 #endif
 constexpr int RPS = NS2D_RPASS_PS;
+#ifndef NS2D_RPASS_SPL_PS
+#define NS2D_RPASS_SPL_PS 3
+#endif
 
 // ---------------------------------------------------------------------------
 // rpass: row pass in (x, ky) space, one row pair (x0, x0+1) per TLR threads
@@ -633,20 +639,24 @@ __device__ __forceinline__ int half_lane(int l) { return (l >> 1) + ((l & 1) ? T
 // tw: the row transforms' twiddle set, twh: the half-length line's.  CFL:
 // the instantiation that can reduce the CFL rate (mode RP_CFL); the step's
 // kernels are built without that code.
-template <int NY, int TLR, int PAIRS, int PFR, bool CFL, bool BAND, typename TW, typename TWH>
+template <int NY, int TLR, int PAIRS, int PFX, bool CFL, bool BAND, typename TW, typename TWH>
 __device__ __forceinline__ void rpass_body_tw(const RPassArgs& a, const int blk, const TW& tw, const TWH& twh) {
+  constexpr int PFR = PFX & 7;
+  constexpr bool SPL = (PFX & 16) != 0;   // exchanges of doubles (fft_reg)
+  static_assert(!SPL || PFR == 2 || PFR == 3, "the mirror exchanges need a complex line buffer");
+  constexpr int RS = SPL ? NS2D_RPASS_SPL_PS : RPS;
   constexpr int T = TLR * PAIRS;
   constexpr int H = NY / 2;
   constexpr int E = NY / TLR;
-  constexpr int LS = padx_s<RPS>(NY) + 1;
+  constexpr int LS = padx_s<RS>(NY) + 1;
   constexpr bool BLOCK = TLR > 64;
   constexpr bool SR = PFR >= 2;
   constexpr bool UPF = PFR == 3 || PFR == 4;   // single row, G fields loaded up front
   constexpr bool HLF = PFR >= 4;               // half-length forward transform
-  static_assert(PFR >= 0 && PFR <= 5, "rpass_body_tw takes the load mode alone");
+  static_assert(PFR >= 0 && PFR <= 5, "bad row-pass load mode");
   static_assert(E >= 2 && (BLOCK ? PAIRS == 1 : 64 % TLR == 0), "bad rpass shape");
   static_assert(!SR || PAIRS == 1, "single-row shapes own one row per workgroup");
-  __shared__ double2 lds[PAIRS * LS];
+  __shared__ double lds[PAIRS * LS * (SPL ? 1 : 2)] __attribute__((aligned(16)));
   __shared__ double red[(T + 63) / 64];
   __shared__ double cred[CFL ? (T + 63) / 64 : 1];
 
@@ -655,7 +665,7 @@ __device__ __forceinline__ void rpass_body_tw(const RPassArgs& a, const int blk,
   const int x0 = SR ? blk : 2 * (blk * PAIRS + q);
   const bool valid = x0 < a.nx;   // uniform per block when BLOCK
   const int ld = a.ld;
-  double2* buf = lds + q * LS;
+  double2* buf = reinterpret_cast<double2*>(lds + q * LS * (SPL ? 1 : 2));
 
   // full-length spectrum of A + iB for row x (which: 0 -> u + iv, 1 -> w_x + i w_y,
   // 2 -> w(x) + i w(x+1), 3 -> w(x))
@@ -751,10 +761,10 @@ __device__ __forceinline__ void rpass_body_tw(const RPassArgs& a, const int blk,
       for (int r = 0; r < 2; ++r) {
         double2 z1[E], z2[E];
         build_pre(z1, 0, pre[r]);
-        fft_reg<NY, TLR, +1, BLOCK, RPS>(z1, buf, tw, opaque(l));
+        fft_reg<NY, TLR, +1, BLOCK, RS, SPL>(z1, buf, tw, opaque(l));
         cfl_acc(z1);
         build_pre(z2, 1, pre[r]);
-        fft_reg<NY, TLR, +1, BLOCK, RPS>(z2, buf, tw, opaque(l));
+        fft_reg<NY, TLR, +1, BLOCK, RS, SPL>(z2, buf, tw, opaque(l));
 #pragma unroll
         for (int e = 0; e < E; ++e) {
           const double nl = z1[e].x * z2[e].x + z1[e].y * z2[e].y;   // u*w_x + v*w_y
@@ -767,10 +777,10 @@ __device__ __forceinline__ void rpass_body_tw(const RPassArgs& a, const int blk,
     double2 z1[E], z2[E];
     build(z1, 0, x0, opaque(l));
     if constexpr (UPF) build(z2, 1, x0, opaque(l));   // both field pairs loaded up front
-    fft_reg<NY, TLR, +1, BLOCK, RPS>(z1, buf, tw, opaque(l));
+    fft_reg<NY, TLR, +1, BLOCK, RS, SPL>(z1, buf, tw, opaque(l));
     cfl_acc(z1);
     if constexpr (!UPF) build(z2, 1, x0, opaque(l));
-    fft_reg<NY, TLR, +1, BLOCK, RPS>(z2, buf, tw, opaque(l));
+    fft_reg<NY, TLR, +1, BLOCK, RS, SPL>(z2, buf, tw, opaque(l));
 #pragma unroll
     for (int e = 0; e < E; ++e) w[e] = make_double2(z1[e].x * z2[e].x + z1[e].y * z2[e].y, 0.0);
   } else if ((a.mode & RP_NL) && (BLOCK || valid)) {
@@ -779,10 +789,10 @@ __device__ __forceinline__ void rpass_body_tw(const RPassArgs& a, const int blk,
       const int x = opaque(x0 + r);
       double2 z1[E], z2[E];
       build(z1, 0, x, opaque(l));
-      fft_reg<NY, TLR, +1, BLOCK, RPS>(z1, buf, tw, opaque(l));
+      fft_reg<NY, TLR, +1, BLOCK, RS, SPL>(z1, buf, tw, opaque(l));
       cfl_acc(z1);
       build(z2, 1, x, opaque(l));
-      fft_reg<NY, TLR, +1, BLOCK, RPS>(z2, buf, tw, opaque(l));
+      fft_reg<NY, TLR, +1, BLOCK, RS, SPL>(z2, buf, tw, opaque(l));
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         const double nl = z1[e].x * z2[e].x + z1[e].y * z2[e].y;   // u*w_x + v*w_y
@@ -817,7 +827,7 @@ __device__ __forceinline__ void rpass_body_tw(const RPassArgs& a, const int blk,
     if (BLOCK || valid) {
       double2 z[E];
       build(z, SR ? 3 : 2, x0, opaque(l));
-      fft_reg<NY, TLR, +1, BLOCK, RPS>(z, buf, tw, opaque(l));
+      fft_reg<NY, TLR, +1, BLOCK, RS, SPL>(z, buf, tw, opaque(l));
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         const int y = l + TLR * e;
@@ -854,7 +864,7 @@ __device__ __forceinline__ void rpass_body_tw(const RPassArgs& a, const int blk,
     if constexpr (HLF) {
       rpass_forward_half<NY, TLR, BLOCK, BAND>(w, buf, a, x0, l, twh);
     } else {
-      fft_reg<NY, TLR, -1, BLOCK, RPS>(w, buf, tw, opaque(l));
+      fft_reg<NY, TLR, -1, BLOCK, RS, SPL>(w, buf, tw, opaque(l));
       // k = l + TLR*e <= H: every element below E/2, lane 0's element E/2 (k = H)
 #pragma unroll
       for (int e = 0; e <= E / 2; ++e) {
@@ -865,7 +875,7 @@ __device__ __forceinline__ void rpass_body_tw(const RPassArgs& a, const int blk,
       }
     }
   } else if ((a.mode & RP_NL) && (BLOCK || valid)) {
-    fft_reg<NY, TLR, -1, BLOCK, RPS>(w, buf, tw, opaque(l));
+    fft_reg<NY, TLR, -1, BLOCK, RS, SPL>(w, buf, tw, opaque(l));
     // W[NY-k] for the thread's own k: exchange through the line buffer
 #pragma unroll
     for (int e = 0; e < E; ++e) buf[padx_s<RPS>(l + TLR * e)] = w[e];
@@ -886,7 +896,7 @@ __device__ __forceinline__ void rpass_body_tw(const RPassArgs& a, const int blk,
 
 template <int NY, int TLR, int PAIRS, int PFR, bool CFL, bool BAND>
 __device__ __forceinline__ void rpass_body(const RPassArgs& a, const int blk) {
-  constexpr int PM = PFR & 7;
+  constexpr int PM = PFR & 7, PX = PFR & 23;
   const int l = (int)threadIdx.x % TLR;
   if constexpr ((PFR & 8) != 0) {
     static_assert(PAIRS == 1 && TLR <= 64, "preloaded twiddle powers are for one-wave rows");
@@ -895,17 +905,17 @@ __device__ __forceinline__ void rpass_body(const RPassArgs& a, const int blk) {
     if constexpr (PM >= 4) {
       TwFull<NY / 2, TLR> twh;
       load_twiddles<NY / 2, TLR>(twh, a.tw, half_lane<TLR>(l));
-      rpass_body_tw<NY, TLR, PAIRS, PM, CFL, BAND>(a, blk, tw, twh);
+      rpass_body_tw<NY, TLR, PAIRS, PX, CFL, BAND>(a, blk, tw, twh);
     } else {
-      rpass_body_tw<NY, TLR, PAIRS, PM, CFL, BAND>(a, blk, tw, a.tw);
+      rpass_body_tw<NY, TLR, PAIRS, PX, CFL, BAND>(a, blk, tw, a.tw);
     }
   } else {
     NS2D_TWIDDLES(NY, TLR, tw, a.tw, l)
     if constexpr (PM >= 4) {
       NS2D_TWIDDLES(NY / 2, TLR, twh, a.tw, half_lane<TLR>(l))
-      rpass_body_tw<NY, TLR, PAIRS, PM, CFL, BAND>(a, blk, tw, twh);
+      rpass_body_tw<NY, TLR, PAIRS, PX, CFL, BAND>(a, blk, tw, twh);
     } else {
-      rpass_body_tw<NY, TLR, PAIRS, PM, CFL, BAND>(a, blk, tw, a.tw);
+      rpass_body_tw<NY, TLR, PAIRS, PX, CFL, BAND>(a, blk, tw, a.tw);
     }
   }
 }
@@ -1423,7 +1433,10 @@ __global__ __launch_bounds__(T) void measures_kernel(MeasArgs a) {
 // points per lane and the four fields on four workgroups give the shortest
 // (64x64 114 -> 62 us per step against 16 columns per wave and workgroup, 128x512
 // 104 -> 45); four points per lane once a launch has thousands of columns
-// (128x4096 140 against 151 us).
+// (128x4096 140 against 151 us).  The other defaults that depend on the column
+// count are in kpass_default_variant.  PF = 2 exchanges doubles instead of
+// complex values (fft_reg, SPL): half the LDS, so that two one-column
+// workgroups of 4096 points share a CU.
 #define NS2D_KPASS_VARIANTS(X) \
   X(8, 16, 64, 4, 3, 1, 0, 1, 0) \
   X(8, 16, 64, 1, 3, 1, 0, 1, 0) \
@@ -1530,6 +1543,8 @@ __global__ __launch_bounds__(T) void measures_kernel(MeasArgs a) {
   X(2048, 2, 512, 1, 4, 8, 0, 1, 0) \
   X(2048, 2, 512, 1, 3, 1, 0, 1, 0) \
   X(2048, 2, 512, 1, 3, 1, 0, 1, 1) \
+  X(2048, 1, 256, 1, 3, 1, 0, 1, 0) \
+  X(2048, 1, 256, 2, 3, 1, 0, 1, 0) \
   X(2048, 2, 512, 1, 3, 1, 1, 4, 0) \
   X(2048, 2, 256, 2, 3, 1, 1, 1, 0) \
   X(2048, 2, 256, 1, 3, 1, 1, 1, 0) \
@@ -1541,6 +1556,7 @@ __global__ __launch_bounds__(T) void measures_kernel(MeasArgs a) {
   X(2048, 2, 512, 1, 3, 8, 0, 1, 0) \
   X(4096, 2, 1024, 1, 4, 8, 0, 1, 0) \
   X(4096, 2, 512, 1, 4, 8, 0, 1, 0) \
+  X(4096, 1, 512, 1, 3, 1, 0, 1, 2) \
   X(4096, 2, 1024, 1, 3, 4, 1, 1, 0) \
   X(4096, 2, 512, 1, 3, 1, 1, 1, 0) \
   X(4096, 2, 512, 1, 4, 4, 1, 1, 0) \
@@ -1593,7 +1609,12 @@ struct KVariant {
 // bound by its traffic and whole waves of row pairs win (4096x64 212 against
 // 254, 4096x256 261 against 283, 4096x512 294 against 305): indices 0 and 1 of
 // these lengths, chosen by rpass_default_variant.  256 with the fields loaded up front as well:
-// 46.7 against 47.8.
+// 46.7 against 47.8.  PFR + 16 exchanges doubles instead of complex values
+// (fft_reg, SPL): at 4096 the 37 KB line buffer lets four 256-thread
+// workgroups share a CU instead of two of 512, and 16 points per thread take
+// two exchanges instead of three: 247 -> 217 us per launch (4096 rows, G fields
+// loaded up front), 267 -> 240 with the per-step max|w| of CN-AB4, which rereads
+// G4 and prefers the fields loaded as needed.
 #define NS2D_RPASS_VARIANTS(X) \
   X(8, 1, 64, 1, 0) \
   X(8, 4, 1, 1, 3) \
@@ -1657,6 +1678,8 @@ struct KVariant {
   X(2048, 512, 1, 1, 3) \
   X(2048, 512, 1, 1, 5) \
   X(2048, 256, 1, 1, 5) \
+  X(4096, 256, 1, 2, 19) \
+  X(4096, 256, 1, 1, 18) \
   X(4096, 512, 1, 4, 2) \
   X(4096, 512, 1, 4, 0) \
   X(4096, 256, 1, 1, 0) \
