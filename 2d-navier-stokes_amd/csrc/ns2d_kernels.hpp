@@ -321,26 +321,48 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
 #pragma unroll
         for (int e = 0; e < E; ++e) R[e] = at(hold, L + lq + TL * e);
       }
+      // one loop per filter (uniform), so that no branch separates a thread's
+      // rows: the table's loads are then all in flight together
       const double nrm = ph.norm2;
+      // (0,0) = 0; a slot past the last column holds no mode, and its ky may
+      // lie past the row's end (ky >= ld), where the per-mode filter table
+      // must not be read
+      auto holds = [&](int e) -> bool { return colv && in_disk(e) && !(kq == 0 && lq + TL * e == 0); };
+      auto scaled = [&](int e, double factor) {                // solver.c:1005, :1019
+        const double2 v = cscale(factor, cscale(nrm, R[e]));
+        const bool in = holds(e);
+        R[e] = make_double2(in ? v.x : 0.0, in ? v.y : 0.0);
+      };
+      if (a.mode & KP_RAW) {
+        // plain unnormalised forward transform (initial conditions); columns
+        // past the last one are not written
+      } else if (BAND || ph.filter == FILTER_NONE) {
+        const bool kill = BAND && ph.kolm_kill;
 #pragma unroll
-      for (int e = 0; e < E; ++e) {
-        const int kx = kx_of_row(lq + TL * e, nx);
-        double2 v = R[e];
-        if (a.mode & KP_RAW) {
-          // plain unnormalised forward transform (initial conditions)
-        } else if ((kx == 0 && kq == 0) || !colv || !in_disk(e)) {
-          // (0,0) = 0; a slot past the last column holds no mode, and its ky
-          // may lie past the row's end (ky >= ld), where the per-mode filter
-          // table must not be read
-          v = make_double2(0.0, 0.0);
-        } else {
-          v = cscale(nrm, v);                                  // solver.c:1005
-          if constexpr (!BAND) v = cscale(dealias_factor(ph, kx, kq), v);   // solver.c:1019
-          else if (ph.kolm_kill && kx == 0) v = cscale(0.0, v);
-          if (ph.force_on && kx == 0 && kq == ph.force_k)      // solver.c:1022-1027
-            v.x += ph.force_val;
+        for (int e = 0; e < E; ++e) scaled(e, kill && lq + TL * e == 0 ? 0.0 : 1.0);
+      } else if (ph.filter == FILTER_HOULI) {
+        double f[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) f[e] = at(ph.filt_tab, kidx(lq + TL * e, colv ? kq : 0, ld, nx));
+#pragma unroll
+        for (int e = 0; e < E; ++e) scaled(e, f[e]);
+      } else if (ph.filter == FILTER_23) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          const int kx = kx_of_row(lq + TL * e, nx);
+          scaled(e, (double)(kx * kx + kq * kq) >= ph.kmax_sqr || (ph.kolm_kill && kx == 0) ? 0.0 : 1.0);
         }
-        R[e] = v;
+      } else {   // FILTER_HOULI_REF
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          const int q = (kx_of_row(lq + TL * e, nx) == ph.nx / 2) + (kq == ph.ny / 2);
+          scaled(e, q == 0 ? 1.0 : (q == 1 ? ph.houli_edge : ph.houli_corner));
+        }
+      }
+      if (ph.force_on && kq == ph.force_k && colv && !(a.mode & KP_RAW)) {   // solver.c:1022-1027
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+          if (lq + TL * e == 0 && holds(e)) R[e].x += ph.force_val;
       }
     }
     const bool conj_fix = (a.mode & KP_CONJFIX) && kq == 0;
