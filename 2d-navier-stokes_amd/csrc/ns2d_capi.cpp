@@ -135,6 +135,15 @@ int visc_kind_plain(const ns2d_handle* h) {
   return VISC_K2;
 }
 
+// A host table into device memory on the stream whose kernels read it (a copy
+// on the null stream is not ordered with a non-blocking stream, neither before
+// its later kernels nor after those that still read the old contents); returns
+// when the host memory may be reused.
+hipError_t upload(hipStream_t s, void* dst, const void* src, size_t bytes) {
+  const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
+  return e != hipSuccess ? e : hipStreamSynchronize(s);
+}
+
 // Per-mode viscous / drag coefficient of the CN factor for one VISC_* kind,
 // evaluated with the host libm pow exactly as the reference writes it
 // (solver.c:835-850, sys_msr.c:160-175); built on first use.
@@ -160,7 +169,7 @@ const double* lam_table(ns2d_handle* h, int kind) {
   }
   double* d = nullptr;
   if (hipMalloc((void**)&d, sizeof(double) * t.size()) != hipSuccess) return nullptr;
-  if (hipMemcpy(d, t.data(), sizeof(double) * t.size(), hipMemcpyHostToDevice) != hipSuccess) {
+  if (upload(h->stream, d, t.data(), sizeof(double) * t.size()) != hipSuccess) {
     (void)hipFree(d);
     return nullptr;
   }
@@ -608,7 +617,7 @@ static int create_impl(const ns2d_params* p, hipStream_t ext_stream, ns2d_t** ou
   }
   if (hipMalloc((void**)&h->tw, sizeof(double2) * NS2D_TW_LEN) != hipSuccess)
     return cleanup(fail(NS2D_ERR_HIP, "hipMalloc failed"));
-  if (hipMemcpy(h->tw, tw.data(), sizeof(double2) * NS2D_TW_LEN, hipMemcpyHostToDevice) != hipSuccess)
+  if (upload(h->stream, h->tw, tw.data(), sizeof(double2) * NS2D_TW_LEN) != hipSuccess)
     return cleanup(fail(NS2D_ERR_HIP, "twiddle upload failed"));
   // Hou-Li filter in its real-division form: per-mode table (solver.c:1088)
   ph.ld = h->ld;
@@ -621,7 +630,7 @@ static int create_impl(const ns2d_params* p, hipStream_t ext_stream, ns2d_t** ou
                                                                         std::pow(j / (p->ny / 2.0), 2.0)), 36.0));
     }
     if (hipMalloc((void**)&h->filt_tab, sizeof(double) * t.size()) != hipSuccess ||
-        hipMemcpy(h->filt_tab, t.data(), sizeof(double) * t.size(), hipMemcpyHostToDevice) != hipSuccess)
+        upload(h->stream, h->filt_tab, t.data(), sizeof(double) * t.size()) != hipSuccess)
       return cleanup(fail(NS2D_ERR_HIP, "filter table upload failed"));
     ph.filt_tab = h->filt_tab;
   }
@@ -747,6 +756,7 @@ int ns2d_set_state_device(ns2d_t* h, const void* d) { return set_state_impl(h, d
 int ns2d_get_state_device(ns2d_t* h, void* d) { return get_state_impl(h, d, hipMemcpyDeviceToDevice); }
 
 static void drop_graph(ns2d_handle* h) {
+  if (h->gexec && h->stream) (void)hipStreamSynchronize(h->stream);   // a replay may still be running
   if (h->gexec) (void)hipGraphExecDestroy(h->gexec);
   if (h->graph) (void)hipGraphDestroy(h->graph);
   h->gexec = nullptr;
@@ -1212,6 +1222,7 @@ struct ns2d_ensemble {
 namespace {
 
 void ens_drop(ns2d_ensemble* e) {
+  if (e->gexec) (void)hipStreamSynchronize(e->stream);   // a replay may still be running
   if (e->gexec) (void)hipGraphExecDestroy(e->gexec);
   if (e->graph) (void)hipGraphDestroy(e->graph);
   e->gexec = nullptr;
@@ -1264,8 +1275,8 @@ int ens_tables(ns2d_ensemble* e, bool check) {
     }
     if (!c.dk) HIPCHK(hipMalloc((void**)&c.dk, sizeof(KPassArgs) * hk.size()));
     if (!c.dr) HIPCHK(hipMalloc((void**)&c.dr, sizeof(RPassArgs) * hr.size()));
-    HIPCHK(hipMemcpy(c.dk, hk.data(), sizeof(KPassArgs) * hk.size(), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(c.dr, hr.data(), sizeof(RPassArgs) * hr.size(), hipMemcpyHostToDevice));
+    HIPCHK(upload(e->stream, c.dk, hk.data(), sizeof(KPassArgs) * hk.size()));
+    HIPCHK(upload(e->stream, c.dr, hr.data(), sizeof(RPassArgs) * hr.size()));
   }
   e->tables_ok = true;
   e->tables_parity = par;
@@ -1977,7 +1988,10 @@ int vjp_impl(ns2d_handle* h, double dt, long n, long ckpt_every, double2** res) 
         g = &c;
     if (!g) {
       g = !h->adj_graph[0].exec ? &h->adj_graph[0] : !h->adj_graph[1].exec ? &h->adj_graph[1] : &h->adj_graph[seg & 1];
-      if (g->exec) (void)hipGraphExecDestroy(g->exec);
+      if (g->exec) {
+        HIPCHK(hipStreamSynchronize(h->stream));   // a replay may still be running
+        (void)hipGraphExecDestroy(g->exec);
+      }
       g->exec = nullptr;
       const int wcur0 = h->wcur, lc0 = lc;
       HIPCHK(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
