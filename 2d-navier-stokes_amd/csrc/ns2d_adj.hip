@@ -6,26 +6,35 @@ namespace ns2d {
 
 // adjoint pass shapes per transform length; index 0 is the default, others
 // are selectable (NS2D_KADJ_VARIANT_<N>, NS2D_RADJ_VARIANT_<N>) for tuning.
-// Row pass {NY, TLR, PAIRS, SR}: SR = 1 runs one row per TLR threads.
+// Row pass {NY, TLR, PAIRS, SR}: SR = 1 runs one row per TLR threads, on two
+// teams up to 64 threads (adj_row_teams); column pass {L, C, T}: C columns per
+// T threads, on four teams up to 64 threads and 1024 points (adj_col_teams).
+// One vector-Jacobian step, forward steps included (us), against the shapes
+// without teams: 64^2 182 -> 78, 128^2 192 -> 84, 256^2 137 -> 102, 512^2
+// 200 -> 172; at 1024 a team's 16 points per lane cost more than they give (column
+// pass 434, one column per 256 threads 350, two per 512 378; row pass of two
+// one-wave teams 437).
 #define NS2D_RADJ_VARIANTS(X) \
+  X(8, 4, 1, 1)        \
   X(8, 1, 64, 0)       \
+  X(16, 8, 1, 1)       \
   X(16, 1, 64, 0)      \
+  X(32, 16, 1, 1)      \
   X(32, 4, 16, 0)      \
+  X(64, 16, 1, 1)      \
   X(64, 8, 8, 0)       \
+  X(128, 64, 1, 1)     \
   X(128, 32, 2, 0)     \
   X(128, 16, 4, 0)     \
   X(256, 64, 1, 1)     \
   X(256, 64, 1, 0)     \
-  X(256, 16, 4, 0)     \
   X(256, 32, 2, 0)     \
   X(512, 64, 1, 1)     \
   X(512, 64, 1, 0)     \
-  X(512, 128, 1, 0)    \
   X(512, 32, 2, 0)     \
   X(1024, 256, 1, 1)   \
   X(1024, 256, 1, 0)   \
   X(1024, 64, 1, 0)    \
-  X(1024, 128, 1, 0)   \
   X(2048, 256, 1, 0)   \
   X(2048, 128, 1, 0)   \
   X(2048, 512, 1, 0)   \
@@ -34,26 +43,26 @@ namespace ns2d {
 
 #define NS2D_KADJ_VARIANTS(X) \
   X(8, 16, 64)       \
+  X(16, 8, 64)       \
   X(16, 16, 64)      \
+  X(32, 4, 64)       \
   X(32, 16, 64)      \
+  X(64, 2, 64)       \
   X(64, 16, 64)      \
+  X(128, 1, 64)      \
   X(128, 16, 128)    \
   X(128, 8, 128)     \
-  X(256, 4, 256)     \
-  X(256, 4, 128)     \
-  X(256, 8, 128)     \
   X(256, 1, 64)      \
+  X(256, 4, 256)     \
+  X(256, 8, 128)     \
   X(256, 1, 128)     \
+  X(512, 1, 64)      \
   X(512, 2, 256)     \
-  X(512, 2, 128)     \
-  X(512, 4, 128)     \
   X(512, 4, 256)     \
   X(512, 1, 128)     \
-  X(512, 1, 64)      \
+  X(1024, 1, 256)    \
   X(1024, 2, 512)    \
   X(1024, 2, 256)    \
-  X(1024, 2, 128)    \
-  X(1024, 1, 256)    \
   X(1024, 1, 128)    \
   X(2048, 2, 512)    \
   X(2048, 2, 256)    \
@@ -102,7 +111,8 @@ hipError_t launch_rpass_adj(int nx, int ny, const RAdjArgs& a, hipStream_t s) {
   }
   if (!v) return hipErrorInvalidValue;
   const int units = v->SR ? nx : nx / 2;   // rows or row pairs
-  hipLaunchKernelGGL(v->kern[a.band ? 1 : 0], dim3((units + v->PAIRS - 1) / v->PAIRS), dim3(v->TLR * v->PAIRS), 0, s, a);
+  hipLaunchKernelGGL(v->kern[a.band ? 1 : 0], dim3((units + v->PAIRS - 1) / v->PAIRS),
+                     dim3(v->TLR * v->PAIRS * adj_row_teams(v->TLR, v->SR)), 0, s, a);
   return hipGetLastError();
 }
 
@@ -122,7 +132,7 @@ hipError_t launch_kpass_adj(int nx, const KAdjArgs& a, hipStream_t s) {
     }
   }
   if (!v) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(v->kern, dim3((a.nyf + v->C - 1) / v->C), dim3(v->T), 0, s, a);
+  hipLaunchKernelGGL(v->kern, dim3((a.nyf + v->C - 1) / v->C), dim3(v->T * adj_col_teams(v->L, v->T)), 0, s, a);
   return hipGetLastError();
 }
 

@@ -60,6 +60,16 @@ namespace ns2d {
 
 __device__ __forceinline__ int kx_of_row(int i, int nx) { return i <= nx / 2 ? i : i - nx; }
 
+// c ? a : b of two pointers, kept as a select: two entries of a kernel
+// argument's pointer array chosen by a lane's value would otherwise be turned
+// into an indexed copy of the array in scratch memory.
+template <typename T>
+__device__ __forceinline__ T* pick(bool c, T* a, T* b) {
+  unsigned long long x = (unsigned long long)a, y = (unsigned long long)b;
+  asm volatile("" : "+v"(x), "+v"(y));
+  return (T*)(c ? x : y);
+}
+
 // Returns v unchanged but opaque to the optimiser.  Used at the top of the
 // per-field / per-batch loops so that index and twiddle arithmetic is redone in
 // each iteration instead of being hoisted and kept live across the loop (which
@@ -1044,8 +1054,13 @@ __global__ __launch_bounds__(TLR * PAIRS, W) void rpass_batched(const RPassArgs*
 // kx parts, the RK4CN adjoint recursion and r2c^T of the next stage.
 // SR = 1: TLR threads own one row (l_n of that row transformed alone, with a
 // zero imaginary part) instead of a row pair: twice the workgroups, five
-// transforms per workgroup instead of nine.
+// transforms per workgroup instead of nine.  A single row of up to 64 threads
+// runs on two teams of TLR threads (adj_row_teams): both transform l_n, one
+// (u, v) and the products' first pair, the other (w_x, w_y) and the second,
+// after they have passed v and w_x across, so that three transforms follow one
+// another instead of five.
 // ---------------------------------------------------------------------------
+constexpr int adj_row_teams(int TLR, int SR) { return SR && TLR <= 64 ? 2 : 1; }
 // BAND: the l_n transform and the G fields reach a.nyc columns (2/3 filter);
 // the products' transforms are wanted in every column (the gradient is not
 // band-limited).
@@ -1057,13 +1072,14 @@ __device__ __forceinline__ void rpass_adj_body(const RAdjArgs& a, const int blk)
   constexpr bool BLOCK = TLR > 64;
   static_assert(E >= 2 && (BLOCK ? PAIRS == 1 : 64 % TLR == 0), "bad rpass_adj shape");
   static_assert(!SR || PAIRS == 1, "single-row shapes own one row per workgroup");
-  __shared__ double2 lds[PAIRS * LS];
+  constexpr int TEAMS = adj_row_teams(TLR, SR);
+  __shared__ double2 lds[PAIRS * TEAMS * LS];
 
   const int tid = threadIdx.x;
-  const int q = tid / TLR, l = tid % TLR;
+  const int q = tid / TLR, l = tid % TLR;   // q: the row pair, or the team
   const int x0 = SR ? blk : 2 * (blk * PAIRS + q);
   const bool valid = x0 < a.nx;
-  if (!BLOCK && !valid) return;
+  if (!BLOCK && !SR && !valid) return;      // (single rows: the grid is nx rows)
   const int ld = a.ld;
   double2* buf = lds + q * LS;
   NS2D_TWIDDLES(NY, TLR, tw, a.tw, l)
@@ -1123,6 +1139,29 @@ __device__ __forceinline__ void rpass_adj_body(const RAdjArgs& a, const int blk)
   double2 zl[E];
   if constexpr (SR) build(zl, a.lin, x0, nullptr, x0, 0, 0, opaque(l), 0);
   else build(zl, a.lin, x0, a.lin, x0 + 1, 0, 0, opaque(l));
+  if constexpr (TEAMS == 2) {
+    double2 z[E];
+    build(z, pick(q != 0, a.g[2], a.g[0]), x0, pick(q != 0, a.g[3], a.g[1]), x0, q ? 0 : 1, q ? 1 : 0, opaque(l));
+    fft_reg<NY, TLR, +1, BLOCK, RPS>(zl, buf, tw, opaque(l));
+    fft_reg<NY, TLR, +1, BLOCK, RPS>(z, buf, tw, opaque(l));
+    // team 0 holds (u, v) and gives v, team 1 holds (w_x, w_y) and gives w_x
+    double* const mine = reinterpret_cast<double*>(buf);
+    const double* const other = reinterpret_cast<const double*>(lds + (1 - q) * LS);
+#pragma unroll
+    for (int e = 0; e < E; ++e) mine[l + TLR * e] = q ? z[e].x : z[e].y;
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const double ln = zl[e].x, o = other[l + TLR * e];
+      z[e] = q ? make_double2(ln * z[e].y, ln * o)     // l_n w_y + i l_n v
+               : make_double2(ln * o, ln * z[e].x);    // l_n w_x + i l_n u
+    }
+    __syncthreads();
+    fft_reg<NY, TLR, -1, BLOCK, RPS>(z, buf, tw, opaque(l));
+    split_store(z, pick(q != 0, a.bout[2], a.bout[0]), pick(q != 0, a.bout[3], a.bout[1]), x0, q ? 0 : 1, q ? 1 : 0,
+                opaque(l));
+    return;
+  }
   fft_reg<NY, TLR, +1, BLOCK, RPS>(zl, buf, tw, opaque(l));
 #pragma unroll 1
   for (int r = 0; r < (SR ? 1 : 2); ++r) {
@@ -1147,20 +1186,29 @@ __device__ __forceinline__ void rpass_adj_body(const RAdjArgs& a, const int blk)
 }
 
 template <int NY, int TLR, int PAIRS, int SR, bool BAND = false>
-__global__ __launch_bounds__(TLR * PAIRS) void rpass_adj_kernel(RAdjArgs a) {
+__global__ __launch_bounds__(TLR * PAIRS * adj_row_teams(TLR, SR)) void rpass_adj_kernel(RAdjArgs a) {
   rpass_adj_body<NY, TLR, PAIRS, SR, BAND>(a, xcd_remap((int)blockIdx.x, (int)gridDim.x));
 }
 
+// Column pass of the adjoint: C columns per group of T threads.  A group that
+// fits a wave (lines of up to 1024 points) runs as four teams of T threads, one
+// per field: the four forward transforms side by side, their sum through LDS,
+// the recursion and the inverse transform on the first team, whose loads of
+// the recursion's arrays are issued before its transform.  Larger groups take
+// the four fields one after another.
+constexpr int adj_col_teams(int L, int T) { return T <= 64 && L <= 1024 ? 4 : 1; }
+
 template <int L, int C, int T>
-__global__ __launch_bounds__(T) void kpass_adj_kernel(KAdjArgs a) {
+__global__ __launch_bounds__(T * adj_col_teams(L, T)) void kpass_adj_kernel(KAdjArgs a) {
   constexpr int TL = T / C;
   constexpr int E = L / TL;
   constexpr int LS = line_stride(L);
   constexpr bool BLOCK = T > 64;
+  constexpr int TEAMS = adj_col_teams(L, T);
   static_assert(T % C == 0 && L % TL == 0 && E >= 2, "bad kpass_adj shape");
-  __shared__ double2 lds[C * LS];
+  __shared__ double2 lds[TEAMS * C * LS];
 
-  const int tid = threadIdx.x;
+  const int team = (int)threadIdx.x / T, tid = (int)threadIdx.x % T;
   const int g = xcd_remap((int)blockIdx.x, (int)gridDim.x);
   const int ky0 = g * C;
   const int c = tid % C, l = tid / C;
@@ -1168,90 +1216,112 @@ __global__ __launch_bounds__(T) void kpass_adj_kernel(KAdjArgs a) {
   const int nyf = a.nyf, ld = a.ld, nx = L;
   const bool colv = ky < nyf;
   const PhysArgs& ph = a.ph;
-  double2* buf = lds + c * LS;
+  double2* buf = lds + (team * C + c) * LS;
   const double h = a.dt;
   NS2D_TWIDDLES(L, TL, tw, a.tw, l)
+  const bool inv_on = (a.mode & KA_INV) != 0;
+  const bool need_acc = a.epi != ADJ_START;
+  const bool need_prev = a.epi == ADJ_S1 && inv_on;
+
+  // the recursion's arrays (a slot past the last column reads column 0 and
+  // writes nothing); the previous step's table in the place of this step's,
+  // which stage 1 does not use
+  constexpr int EP = TEAMS == 4 ? E : 1;
+  double2 lp[EP], ac[EP];
+  double lm[EP];
+  auto load_epi = [&](int e, int slot) {
+    const size_t idx = kidx(l + TL * e, colv ? ky : 0, ld, nx);
+    lp[slot] = at(a.lamp_in, idx);
+    ac[slot] = need_acc ? at(a.lacc, idx) : make_double2(0.0, 0.0);
+    lm[slot] = at(need_prev ? a.lam_prev : a.lam, idx);
+  };
+  // conj(U) = 1/|k|^2 (-i ky in B1), conj(X) = -i kx, conj(V) = i kx/|k|^2, conj(Y): -i ky in B4
+  auto term = [&](int f, int x, double2 v, int kyv) -> double2 {
+    const int kx = kx_of_row(x, nx);
+    if (f == 3) return v;
+    if (f == 1) return make_double2(kx * v.y, -kx * v.x);
+    const int k2i = kx * kx + kyv * kyv;
+    const double inv = k2i ? rcp_nr((double)k2i) : 0.0;
+    if (f == 0) return cscale(inv, v);
+    return make_double2(-(kx * inv) * v.y, (kx * inv) * v.x);
+  };
 
   double2 LSacc[E];   // N'(S)^T l_K of the stage just finished
 #pragma unroll
   for (int e = 0; e < E; ++e) LSacc[e] = make_double2(0.0, 0.0);
-  if (a.mode & KA_FWD) {
-#pragma unroll 1
-    for (int f = 0; f < 4; ++f) {
-      const int l_o = opaque(l), ky_o = opaque(ky);
+  if constexpr (TEAMS == 4) {
+    if (team == 0) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) load_epi(e, TEAMS == 4 ? e : 0);
+    }
+    if (a.mode & KA_FWD) {
+      const double2* const in = pick(team >= 2, pick(team == 3, a.bin[3], a.bin[2]), pick(team == 1, a.bin[1], a.bin[0]));
       double2 F[E];
 #pragma unroll
-      for (int e = 0; e < E; ++e) {
-        F[e] = colv ? a.bin[f][nidx(l_o + TL * e, ky_o, ld)] : make_double2(0.0, 0.0);
-        if ((e & 3) == 3) asm volatile("" ::: "memory");
-      }
-      fft_reg<L, TL, -1, BLOCK>(F, buf, tw, l_o);
+      for (int e = 0; e < E; ++e) F[e] = at(in, nidx(l + TL * e, colv ? ky : 0, ld));
+      fft_reg<L, TL, -1, BLOCK>(F, buf, tw, opaque(l));
+      if (team != 0) {
 #pragma unroll
-      for (int e = 0; e < E; ++e) {
-        const int kx = kx_of_row(l_o + TL * e, nx);
-        const int k2i = kx * kx + ky_o * ky_o;
-        const double inv = k2i ? rcp_nr((double)k2i) : 0.0;
-        const double2 v = F[e];
-        double2 t;
-        if (f == 0) t = cscale(inv, v);                                   // conj(U): 1/|k|^2 (-i ky in B1)
-        else if (f == 1) t = make_double2(kx * v.y, -kx * v.x);          // conj(X) = -i kx
-        else if (f == 2) t = make_double2(-(kx * inv) * v.y, (kx * inv) * v.x);  // conj(V) = i kx/|k|^2
-        else t = v;                                                       // conj(Y): -i ky in B4
-        LSacc[e] = cadd(LSacc[e], t);
+        for (int e = 0; e < E; ++e) buf[padx(l + TL * e)] = term(team, l + TL * e, F[e], ky);
+      }
+      __syncthreads();
+      if (team == 0) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          const int p = c * LS + padx(l + TL * e);
+          LSacc[e] = cadd(cadd(cadd(term(0, l + TL * e, F[e], ky), lds[C * LS + p]), lds[2 * C * LS + p]), lds[3 * C * LS + p]);
+        }
+      }
+    }
+    if (team != 0) return;
+  } else {
+    if (a.mode & KA_FWD) {
+#pragma unroll 1
+      for (int f = 0; f < 4; ++f) {
+        const int l_o = opaque(l), ky_o = opaque(ky);
+        double2 F[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          F[e] = at(a.bin[f], nidx(l_o + TL * e, colv ? ky_o : 0, ld));
+          if ((e & 3) == 3) asm volatile("" ::: "memory");
+        }
+        fft_reg<L, TL, -1, BLOCK>(F, buf, tw, l_o);
+#pragma unroll
+        for (int e = 0; e < E; ++e) LSacc[e] = cadd(LSacc[e], term(f, l_o + TL * e, F[e], ky_o));
       }
     }
   }
 
   // RK4CN adjoint recursion (backwards through solver.c:690-853)
+  // l_K4 = mu/6, l_K3 = mu/3 + h l_S4, l_K2 = mu/3 + (h/2) l_S3, l_K1 = mu/6 + (h/2) l_S2
+  const double bw = (a.epi == ADJ_S4 || a.epi == ADJ_S3) ? RK4_B2 : RK4_B1;
+  const double cw = a.epi == ADJ_S4 ? h : 0.5 * h;
   double2 LK[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) {
-    LK[e] = make_double2(0.0, 0.0);
-    if (!colv) continue;
-    const int kx = kx_of_row(l + TL * e, nx);
-    const size_t idx = kidx(l + TL * e, ky, ld, nx);
-    const bool zero = (kx == 0 && ky == 0);
-    const double D = h * a.lam[idx];
+    const int x = l + TL * e;
+    const size_t idx = kidx(x, colv ? ky : 0, ld, nx);
+    const bool zero = x == 0 && ky == 0;
+    const int slot = TEAMS == 4 ? e : 0;
+    if constexpr (TEAMS != 4) load_epi(e, 0);
+    const double D = h * lm[slot];
     const double q = rcp_nr(2.0 + D);
     const double A = (2.0 - D) * q, B = 2.0 * h * q;
-    double2 lp = a.lamp_in[idx];   // dJ/dw_{n+1}
-    if (zero) lp = make_double2(0.0, 0.0);
-    switch (a.epi) {
-      case ADJ_START:
-        a.lacc[idx] = cscale(A, lp);
-        LK[e] = cscale(B * RK4_B1, lp);
-        break;
-      case ADJ_S4:
-        a.lacc[idx] = cadd(a.lacc[idx], LSacc[e]);
-        LK[e] = cadd(cscale(B * RK4_B2, lp), cscale(h, LSacc[e]));
-        break;
-      case ADJ_S3:
-        a.lacc[idx] = cadd(a.lacc[idx], LSacc[e]);
-        LK[e] = cadd(cscale(B * RK4_B2, lp), cscale(0.5 * h, LSacc[e]));
-        break;
-      case ADJ_S2:
-        a.lacc[idx] = cadd(a.lacc[idx], LSacc[e]);
-        LK[e] = cadd(cscale(B * RK4_B1, lp), cscale(0.5 * h, LSacc[e]));
-        break;
-      case ADJ_S1: {
-        // dJ/dw_n; with KA_INV it starts the adjoint of the previous step
-        const double2 lw = cadd(a.lacc[idx], LSacc[e]);
-        a.lamp_out[idx] = lw;
-        if (a.mode & KA_INV) {
-          const double Dp = h * a.lam_prev[idx];
-          const double qp = rcp_nr(2.0 + Dp);
-          const double Ap = (2.0 - Dp) * qp, Bp = 2.0 * h * qp;
-          const double2 lq = zero ? make_double2(0.0, 0.0) : lw;
-          a.lacc[idx] = cscale(Ap, lq);
-          LK[e] = cscale(Bp * RK4_B1, lq);
-        }
-        break;
-      }
-      default: break;
+    const double2 sum = cadd(ac[slot], LSacc[e]);
+    // dJ/dw at the end of the step whose recursion this is: dJ/dw_{n+1}, at
+    // stage 1 the dJ/dw_n just finished, which starts the previous step
+    const double2 src = a.epi == ADJ_S1 ? sum : lp[slot];
+    const double2 lw = make_double2(zero ? 0.0 : src.x, zero ? 0.0 : src.y);
+    const double2 mu = cscale(B * bw, lw);
+    const bool starts = a.epi == ADJ_START || a.epi == ADJ_S1;
+    LK[e] = starts ? mu : cadd(mu, cscale(cw, LSacc[e]));
+    if (colv) {
+      if (a.epi == ADJ_S1) at(a.lamp_out, idx) = sum;
+      if (a.epi != ADJ_S1 || inv_on) at(a.lacc, idx) = starts ? cscale(A, lw) : sum;
     }
-    if ((e & 3) == 3) asm volatile("" ::: "memory");
+    if (TEAMS != 4 && (e & 3) == 3) asm volatile("" ::: "memory");
   }
-  if (!(a.mode & KA_INV)) return;
+  if (!inv_on) return;
   // a column the filter zeroes entirely has a zero l_n transform, which the
   // band-limited row pass does not read
   if (ky0 >= a.nyc) return;
@@ -1270,7 +1340,7 @@ __global__ __launch_bounds__(T) void kpass_adj_kernel(KAdjArgs a) {
     fft_reg<L, TL, +1, BLOCK>(LK, buf, tw, l_o);
     if (colv) {
 #pragma unroll
-      for (int e = 0; e < E; ++e) a.lout[gidx(l_o + TL * e, ky_o, ld)] = LK[e];
+      for (int e = 0; e < E; ++e) at(a.lout, gidx(l_o + TL * e, ky_o, ld)) = LK[e];
     }
   }
 }
