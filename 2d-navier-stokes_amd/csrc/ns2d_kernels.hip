@@ -290,27 +290,59 @@ hipError_t launch_r2c_rows(int nx, int ny, const double* in, double2* out, const
 // they are zero and not read (NaN once the state has blown up: a NaN in any
 // mode has then reached every mode of the disk, and 0 * NaN is what the
 // filter leaves).
+// A transpose for the column-major layout: 32 x 32 tiles through LDS (rows one
+// 16-B slot longer than the tile, so that a column's reads fall on distinct
+// banks), both sides in runs of 512 B.  Bound by memory: 2 x 16 B per mode.
+constexpr int RELAYOUT_TILE = 32;
 __global__ __launch_bounds__(256) void relayout_kernel(const double2* __restrict__ src, double2* __restrict__ dst,
                                                        int nyf, int ld, int nx, int dir, long kc2,
                                                        unsigned long long* __restrict__ spill,
                                                        unsigned long long epoch) {
-  const int x = blockIdx.y, ky = blockIdx.x * 256 + threadIdx.x;
+  constexpr int RT = RELAYOUT_TILE, ROWS = 256 / RT;
+  __shared__ double2 tile[RT][RT + 1];   // [x][ky]
+  const int x0 = (int)blockIdx.y * RT, k0 = (int)blockIdx.x * RT;
+  const int tx = (int)threadIdx.x % RT, ty = (int)threadIdx.x / RT;
+  auto outside = [&](int x, int ky) -> bool {
+    const long kx = kx_of_row(x, nx);
+    return kc2 > 0 && kx * kx + (long)ky * ky >= kc2;
+  };
   if (dir == 0) {
-    const double2 v = ky < nyf ? src[(size_t)x * nyf + ky] : make_double2(0.0, 0.0);
-    if (ky < ld) dst[kidx(x, ky, ld, nx)] = v;
-    const long kx = kx_of_row(x, nx);
-    if (kc2 > 0 && kx * kx + (long)ky * ky >= kc2 && !(v.x == 0.0 && v.y == 0.0)) *spill = epoch;
-  } else if (ky < nyf) {
-    const long kx = kx_of_row(x, nx);
-    const bool out = kc2 > 0 && kx * kx + (long)ky * ky >= kc2;
-    const double2 v = src[out ? kidx(1, 0, ld, nx) : kidx(x, ky, ld, nx)];
-    dst[(size_t)x * nyf + ky] = out ? cscale(0.0, v) : v;
+    bool spills = false;
+#pragma unroll
+    for (int r = ty; r < RT; r += ROWS) {
+      const int x = x0 + r, ky = k0 + tx;
+      const bool in = x < nx && ky < nyf;
+      const double2 v = in ? src[(size_t)x * nyf + ky] : make_double2(0.0, 0.0);
+      spills = spills || (in && outside(x, ky) && !(v.x == 0.0 && v.y == 0.0));
+      tile[r][tx] = v;
+    }
+    if (spills) *spill = epoch;
+    __syncthreads();
+#pragma unroll
+    for (int r = ty; r < RT; r += ROWS) {
+      const int x = x0 + tx, ky = k0 + r;
+      if (x < nx && ky < ld) dst[kidx(x, ky, ld, nx)] = tile[tx][r];
+    }
+  } else {
+    const double2 z = cscale(0.0, src[kidx(1, 0, ld, nx)]);
+#pragma unroll
+    for (int r = ty; r < RT; r += ROWS) {
+      const int x = x0 + tx, ky = k0 + r;
+      if (x < nx && ky < nyf) tile[tx][r] = outside(x, ky) ? z : src[kidx(x, ky, ld, nx)];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = ty; r < RT; r += ROWS) {
+      const int x = x0 + r, ky = k0 + tx;
+      if (x < nx && ky < nyf) dst[(size_t)x * nyf + ky] = tile[r][tx];
+    }
   }
 }
 
 hipError_t launch_relayout(const double2* src, double2* dst, int nx, int nyf, int ld, int dir, long kc2,
                            unsigned long long* spill, unsigned long long epoch, hipStream_t s) {
-  hipLaunchKernelGGL(relayout_kernel, dim3((ld + 255) / 256, nx), dim3(256), 0, s, src, dst, nyf, ld, nx, dir, kc2, spill, epoch);
+  constexpr int RT = RELAYOUT_TILE;
+  hipLaunchKernelGGL(relayout_kernel, dim3((ld + RT - 1) / RT, (nx + RT - 1) / RT), dim3(256), 0, s, src, dst, nyf, ld, nx, dir, kc2, spill, epoch);
   return hipGetLastError();
 }
 
