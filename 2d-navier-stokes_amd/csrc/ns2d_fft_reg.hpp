@@ -271,7 +271,19 @@ __device__ __forceinline__ void apply_butterfly_twiddles(double2* x, const TwFul
 // line buffer of N doubles (padded like the complex one), for shapes whose
 // workgroups per CU are limited by LDS: half the buffer, two barriers more per
 // exchange.
-template <int N, int TL, int SIGN, bool BLOCK, int P, int PS, int OFF, bool SPL, typename TW>
+// DB > 0: exchanges alternate between two line buffers DB slots apart, so that
+// none has to wait until all threads have read the one before (one barrier per
+// exchange instead of two); the number of exchanges must be even, so that the
+// next transform may start on the first buffer again.
+template <int N, int TL>
+constexpr int fft_exchanges() {
+  constexpr int E = N / TL, R = E < 16 ? E : 16;
+  int n = 0;
+  for (int p = R; p < N; p *= R) ++n;
+  return n;
+}
+
+template <int N, int TL, int SIGN, bool BLOCK, int P, int PS, int OFF, bool SPL, int DB, typename TW>
 __device__ __forceinline__ void fft_reg_pass(double2* v, double2* buf, const TW& tw, int l) {
   constexpr int E = N / TL;
   constexpr int REM = N / P;
@@ -329,9 +341,9 @@ __device__ __forceinline__ void fft_reg_pass(double2* v, double2* buf, const TW&
 #pragma unroll
         for (int e = 0; e < E; ++e) v[e] = buf[fft_slot<PS, P, R>(l + TL * e)];
       }
-      xsync<BLOCK>();
+      if constexpr (DB == 0) xsync<BLOCK>();
       fft_reg_pass<N, TL, SIGN, BLOCK, P * R, PS,
-                   OFF + (P > 1 ? NB * TwSlots<TW>::template per_butterfly<R>() : 0), SPL>(v, buf, tw, l);
+                   OFF + (P > 1 ? NB * TwSlots<TW>::template per_butterfly<R>() : 0), SPL, -DB>(v, buf + DB, tw, l);
     }
   }
 }
@@ -342,11 +354,12 @@ __device__ __forceinline__ void fft_reg_pass(double2* v, double2* buf, const TW&
 // must call.
 // tw: the global table (const double2*) or the thread's preloaded TwReg<N, TL>
 // (loaded with the same l).  SPL: buf holds padx_s<PS>(N) doubles.
-template <int N, int TL, int SIGN, bool BLOCK, int PS = 3, bool SPL = false, typename TW>
+template <int N, int TL, int SIGN, bool BLOCK, int PS = 3, bool SPL = false, int DB = 0, typename TW>
 __device__ __forceinline__ void fft_reg(double2* v, double2* buf, const TW& tw, int l) {
   static_assert((N & (N - 1)) == 0 && N >= 2 && N % TL == 0, "bad FFT shape");
   static_assert(N <= NS2D_TW_LEN, "twiddle table too short");
-  fft_reg_pass<N, TL, SIGN, BLOCK, 1, PS, 0, SPL>(v, buf, tw, l);
+  static_assert(DB == 0 || (!SPL && fft_exchanges<N, TL>() % 2 == 0), "two line buffers need an even number of exchanges");
+  fft_reg_pass<N, TL, SIGN, BLOCK, 1, PS, 0, SPL, DB>(v, buf, tw, l);
 }
 
 }  // namespace ns2d

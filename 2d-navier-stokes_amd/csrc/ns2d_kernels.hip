@@ -113,6 +113,8 @@ static int r_index(int NY, int TLR, int PAIRS, int PFR) {
 //   128   > 512 columns   2 columns, 4 points per lane  (128x4096 RK4CN step 140 / 151)
 //   256   > 1024          2 splits instead of 4         2049 columns 21.7 / 26.5
 //   512   > 400           2 columns, 2 splits           513: 21.2 / 22.0, 2049: 37.5 / 53.2
+//   512   <= 400          index 0 on two line buffers   257: 15.1 / 15.7
+//   1024  <= 512          index 0 on two line buffers   341: 22.6 / 23.6 (513: 28.1 / 24.3)
 //   1024  > 700           2 columns of 512 threads      1025: 41.7 / 45.6, 2049: 76.7 / 97.3
 //   2048  <= 300          1 column, 2 splits            257: 27.5 / 34.0
 //   2048  <= 700          1 column                      513: 40.8 / 46.0, 683: 45.7 / 46.7
@@ -120,7 +122,8 @@ static int r_index(int NY, int TLR, int PAIRS, int PFR) {
 int kpass_default_variant(int nx, int nyc) {
   if (nx == 128 && nyc > 512) return k_index(128, 2, 64, 4, 3, 1, 0);
   if (nx == 256 && nyc > 1024) return k_index(256, 1, 64, 2, 3, 1, 0);
-  if (nx == 512 && nyc > 400) return k_index(512, 2, 256, 2, 4, 8, 0);
+  if (nx == 512) return nyc > 400 ? k_index(512, 2, 256, 2, 4, 8, 0) : k_index(512, 1, 128, 4, 3, 1, 4);
+  if (nx == 1024 && nyc <= 512) return k_index(1024, 1, 256, 2, 4, 1, 4);
   if (nx == 1024 && nyc > 700) return k_index(1024, 2, 512, 2, 4, 8, 0);
   if (nx == 2048 && nyc <= 300) return k_index(2048, 1, 256, 2, 3, 1, 0);
   if (nx == 2048 && nyc <= 700) return k_index(2048, 1, 256, 1, 3, 1, 0);
@@ -170,7 +173,8 @@ int kpass_variant_extra(int nx, int idx, int* W, int* PS, int* OFF, int* PK) {
   *W = v->W;
   *PS = v->PS;
   *OFF = v->OFF;
-  *PK = (v->PK != 0) | ((v->PF & 1) << 1) | ((v->PK == 2) << 2) | (((v->PF & 2) != 0) << 6);
+  *PK = (v->PK != 0) | ((v->PF & 1) << 1) | ((v->PK == 2) << 2) | (((v->PF & 2) != 0) << 6) |
+        (((v->PF & 4) != 0) << 7);
   return 0;
 }
 

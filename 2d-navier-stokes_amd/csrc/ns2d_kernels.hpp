@@ -171,14 +171,16 @@ template <int L, int C, int T, int KS, int PS, int OFF, int PK, int PFX, bool BA
 __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
   constexpr int PF = PFX & 1;
   constexpr bool SPL = (PFX & 2) != 0;   // exchanges of doubles (fft_reg)
-  static_assert(!(SPL && PK), "the packed pair needs a complex line buffer");
+  constexpr bool DBL = (PFX & 4) != 0;   // exchanges alternate between two buffers (fft_reg)
+  static_assert(!((SPL || DBL) && PK), "the packed pair needs its one complex line buffer");
   constexpr int TL = T / C;        // threads per column
   constexpr int E = L / TL;        // rows per thread
   constexpr int LS = padx_s<PS>(L) + OFF;
   constexpr int FPS = 4 / KS;      // inverse fields per split
   constexpr bool BLOCK = T > 64;
   static_assert(T % C == 0 && L % TL == 0 && E >= 2 && 4 % KS == 0, "bad kpass shape");
-  __shared__ double lds[C * LS * (SPL ? 1 : 2)] __attribute__((aligned(16)));
+  constexpr int DB = DBL ? C * LS : 0;
+  __shared__ double lds[C * LS * (SPL ? 1 : DBL ? 4 : 2)] __attribute__((aligned(16)));
 
   const int tid = threadIdx.x;
   // a pass without inverse transforms has one work item per column group
@@ -283,7 +285,7 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
       else R[e] = colv ? at(a.nin, nidx(x, ky, ld)) : make_double2(0.0, 0.0);
       if ((e & 3) == 3) asm volatile("" ::: "memory");
     }
-    fft_reg<L, TL, -1, BLOCK, PS, SPL>(R, buf, tw, opaque(l));
+    fft_reg<L, TL, -1, BLOCK, PS, SPL, DB>(R, buf, tw, opaque(l));
     if (pblk) {
       if (pair) {
 #pragma unroll
@@ -583,7 +585,7 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
 #pragma unroll
       for (int e = 0; e < E; ++e) F[e] = derive(f, R[e], kx_of_row(l_o + TL * e, nx), ky_o);
     }
-    fft_reg<L, TL, +1, BLOCK, PS, SPL>(F, buf, tw, l_o);
+    fft_reg<L, TL, +1, BLOCK, PS, SPL, DB>(F, buf, tw, l_o);
     double2* __restrict__ gout = a.g[f];
     if (pair) {
       double* __restrict__ g4 = reinterpret_cast<double*>(a.g[3]);
@@ -1528,7 +1530,11 @@ __global__ __launch_bounds__(T) void measures_kernel(MeasArgs a) {
 // (128x4096 140 against 151 us).  The other defaults that depend on the column
 // count are in kpass_default_variant.  PF = 2 exchanges doubles instead of
 // complex values (fft_reg, SPL): half the LDS, so that two one-column
-// workgroups of 4096 points share a CU.
+// workgroups of 4096 points share a CU.  PF = 4 alternates the exchanges between
+// two line buffers (one barrier each instead of two) where the grid leaves the
+// LDS: 512 points 15.7 -> 15.1 us per launch (257 columns), 13.4 -> 13.0 (171);
+// 1024 points 23.6 -> 22.6 (341 columns), but 24.3 -> 28.1 at 513, whose 1026
+// workgroups need a fifth on two CUs.
 #define NS2D_KPASS_VARIANTS(X) \
   X(8, 16, 64, 4, 3, 1, 0, 1, 0) \
   X(8, 16, 64, 1, 3, 1, 0, 1, 0) \
@@ -1567,6 +1573,7 @@ __global__ __launch_bounds__(T) void measures_kernel(MeasArgs a) {
   X(256, 2, 128, 4, 3, 1, 0, 1, 0) \
   X(256, 1, 128, 4, 3, 1, 0, 1, 0) \
   X(512, 1, 128, 4, 3, 1, 0, 1, 0) \
+  X(512, 1, 128, 4, 3, 1, 0, 1, 4) \
   X(512, 1, 128, 4, 3, 1, 0, 1, 1) \
   X(512, 2, 256, 2, 3, 1, 0, 1, 0) \
   X(512, 4, 256, 2, 3, 1, 0, 1, 0) \
@@ -1591,6 +1598,7 @@ __global__ __launch_bounds__(T) void measures_kernel(MeasArgs a) {
   X(512, 1, 64, 4, 3, 1, 0, 1, 0) \
   X(512, 1, 64, 2, 3, 1, 0, 1, 0) \
   X(1024, 1, 256, 2, 4, 1, 0, 1, 0) \
+  X(1024, 1, 256, 2, 4, 1, 0, 1, 4) \
   X(1024, 1, 256, 2, 3, 1, 0, 1, 0) \
   X(1024, 1, 256, 2, 3, 1, 0, 1, 1) \
   X(1024, 2, 512, 2, 4, 8, 0, 1, 0) \
