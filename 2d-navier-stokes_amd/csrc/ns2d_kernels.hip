@@ -131,24 +131,36 @@ int kpass_default_variant(int nx, int nyc) {
   return 0;
 }
 
-// Default row-pass shape: index 0 of its length, but
-//   up to 128   single rows (index 0 is row pairs in whole waves) for their
-//               shorter chain, below 2048 rows
-//   256, 512    row pairs in whole waves from 2048 rows on, where the pass is
-//               bound by its traffic (figures at NS2D_RPASS_VARIANTS)
-//   1024        from 2048 rows on, the fields loaded as needed: two waves per
-//               SIMD instead of one (2048 rows 27.6 / 30.2 us per launch, 4096
-//               rows 44.4 / 51.5)
-//   4096        up to 512 rows the 512-thread shape (512 rows 22.6 / 23.3);
-//               with CN-AB4's max|w| in every step the fields loaded as needed
+// Default row-pass shape.  Below 2048 rows a launch is one chain of latencies:
+// up to 1024 points a single row on two teams (rpass_team_body).  From 2048 rows
+// on the pass is bound by its traffic:
+//   up to 512   row pairs in whole waves (2048x512 171.6 us per step against 174.0 on
+//               teams, 4096x512 294 / 305, 4096x64 212 / 254)
+//   1024        single rows, the fields loaded as needed: two waves per SIMD
+//               (2048x1024 263.5 / 264.8, 4096 rows 44.4 / 51.5 us per launch)
+// CN-AB4 forms max|w| in every step, which row pairs do with one transform for two
+// rows: 1024 points from 1024 rows on 43.9 us per step against 48.4 (1024^2),
+// 81.3 / 88.1 (2048x1024).  4096: index 0, exchanges of doubles; up to 512 rows the
+// 512-thread shape (22.6 / 23.3 us per launch); with CN-AB4 the fields loaded as
+// needed (443.8 against 463 us per step).
 int rpass_default_variant(int nx, int ny, bool ab4) {
   const bool tall = nx >= 2048;
-  if (ny < 256) return tall ? 0 : 1;   // index 0: row pairs
-  if (ny <= 512) return tall ? 1 : 0;  // index 1: row pairs
-  if (ny == 1024 && tall) return r_index(1024, 64, 1, 2);
-  if (ny == 4096 && nx <= 512) return r_index(4096, 512, 1, 2);
-  if (ny == 4096 && ab4) return r_index(4096, 256, 1, 18);
-  return 0;
+  switch (ny) {
+    case 8: return tall ? 0 : r_index(8, 4, 1, 3);
+    case 16: return tall ? 0 : r_index(16, 8, 1, 3);
+    case 32: return tall ? 0 : r_index(32, 16, 1, 6);
+    case 64: return tall ? 0 : r_index(64, 16, 1, 14);
+    case 128: return tall ? 0 : r_index(128, 64, 1, 14);
+    case 256: return tall ? r_index(256, 32, 2, 0) : r_index(256, 64, 1, 6);
+    case 512: return tall ? r_index(512, 64, 4, 0) : r_index(512, 64, 1, 6);
+    case 1024:
+      if (ab4 && nx >= 1024) return r_index(1024, 256, 1, 1);
+      return tall ? r_index(1024, 64, 1, 2) : r_index(1024, 64, 1, 6);
+    case 4096:
+      if (nx <= 512) return r_index(4096, 512, 1, 2);
+      return ab4 ? r_index(4096, 256, 1, 18) : 0;
+    default: return 0;
+  }
 }
 
 int kpass_variant_count(int nx) {
@@ -214,7 +226,8 @@ hipError_t launch_rpass_batched(int nx, int ny, int band, int variant, const RPa
   if (!v) return hipErrorInvalidValue;
   const int units = (v->PFR & 7) >= 2 ? nx : nx / 2;   // rows or row pairs
   const int per = (units + v->PAIRS - 1) / v->PAIRS;
-  hipLaunchKernelGGL(v->batched[band ? 1 : 0], dim3(per * members), dim3(v->TLR * v->PAIRS), 0, s, tab, per);
+  hipLaunchKernelGGL(v->batched[band ? 1 : 0], dim3(per * members), dim3(v->TLR * v->PAIRS * rpass_teams(v->PFR)), 0, s, tab,
+                     per);
   return hipGetLastError();
 }
 
@@ -241,7 +254,7 @@ int rpass_variant_extra(int ny, int idx, int* W, int* PS, int* OFF, int* PK) {
   *PS = 3;
   *OFF = 1;
   const int pm = v->PFR & 7;
-  *PK = ((pm == 1 || pm == 3 || pm == 4) << 1) | ((pm >= 2) << 3) | ((pm >= 4) << 4) | (((v->PFR & 8) != 0) << 5) |
+  *PK = ((pm == 1 || pm == 3 || pm == 4) << 1) | ((pm >= 2) << 3) | ((pm == 4 || pm == 5 || pm == 7) << 4) | ((pm >= 6) << 8) | (((v->PFR & 8) != 0) << 5) |
         (((v->PFR & 16) != 0) << 6);
   return 0;
 }
@@ -252,7 +265,7 @@ hipError_t launch_rpass(int nx, int ny, int variant, const RPassArgs& a, hipStre
   const int units = (v->PFR & 7) >= 2 ? nx : nx / 2;   // rows or row pairs
   const int b = a.band ? 1 : 0;
   hipLaunchKernelGGL((a.mode & RP_CFL) ? v->cfl[b] : v->kern[b], dim3((units + v->PAIRS - 1) / v->PAIRS),
-                     dim3(v->TLR * v->PAIRS), 0, s, a);
+                     dim3(v->TLR * v->PAIRS * rpass_teams(v->PFR)), 0, s, a);
   return hipGetLastError();
 }
 

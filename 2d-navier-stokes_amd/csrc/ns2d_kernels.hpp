@@ -670,6 +670,49 @@ __device__ __forceinline__ void rpass_forward_half(double2 (&w)[NY / TLR], doubl
 template <int TLR>
 __device__ __forceinline__ int half_lane(int l) { return (l >> 1) + ((l & 1) ? TLR / 2 : 0); }
 
+// full-length spectrum of A + iB for row x (which: 0 -> u + iv, 1 -> w_x + i w_y,
+// 2 -> w(x) + i w(x+1), 3 -> w(x))
+// Element e of lane lo holds ky = lo + TLR*e: elements below E/2 lie in
+// [0, H), those above E/2 in (H, NY), and only lane 0's elements 0 and E/2
+// are the real-valued ky = 0 and ky = H, so the mirror and edge tests are
+// fixed per element once the loop is unrolled.
+template <int NY, int TLR, bool BAND>
+__device__ __forceinline__ void rpass_build(double2 (&z)[NY / TLR], int which, int x, int lo, const RPassArgs& a) {
+  constexpr int E = NY / TLR;
+  const int ld = a.ld;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int ky = lo + TLR * e;
+    const bool edge = (e == 0 || e == E / 2) && lo == 0;
+    const bool mirror = e > E / 2 || (e == E / 2 && lo != 0);
+    const int kk = mirror ? NY - ky : ky;
+    // a column past the band takes column 0's address and then zero
+    const bool in = !BAND || kk < a.nyc;
+    const int kl = in ? kk : 0;
+    double2 A, B;
+    const double fk = (double)kk;
+    if (which == 0) {         // u = i ky G1, v = G2
+      const double2 g1 = at(a.g[0], gidx(x, kl, ld));
+      A = make_double2(-fk * g1.y, fk * g1.x);
+      B = at(a.g[1], gidx(x, kl, ld));
+    } else if (which == 1) {  // w_x = G3, w_y = i ky G4
+      A = at(a.g[2], gidx(x, kl, ld));
+      const double2 g4 = at(a.g[3], gidx(x, kl, ld));
+      B = make_double2(-fk * g4.y, fk * g4.x);
+    } else if (which == 2) {  // w of rows x and x+1 = G4
+      A = at(a.g[3], gidx(x, kl, ld));
+      B = at(a.g[3], gidx(x + 1, kl, ld));
+    } else {                  // w of row x alone
+      A = at(a.g[3], gidx(x, kl, ld));
+      B = make_double2(0.0, 0.0);
+    }
+    if (edge) { A.y = 0.0; B.y = 0.0; }
+    z[e] = mirror ? make_double2(A.x + B.y, B.x - A.y) : make_double2(A.x - B.y, A.y + B.x);
+    if (!in) z[e] = make_double2(0.0, 0.0);
+    if ((e & 3) == 3) asm volatile("" ::: "memory");
+  }
+}
+
 // tw: the row transforms' twiddle set, twh: the half-length line's.  CFL:
 // the instantiation that can reduce the CFL rate (mode RP_CFL); the step's
 // kernels are built without that code.
@@ -701,45 +744,7 @@ __device__ __forceinline__ void rpass_body_tw(const RPassArgs& a, const int blk,
   const int ld = a.ld;
   double2* buf = reinterpret_cast<double2*>(lds + q * LS * (SPL ? 1 : 2));
 
-  // full-length spectrum of A + iB for row x (which: 0 -> u + iv, 1 -> w_x + i w_y,
-  // 2 -> w(x) + i w(x+1), 3 -> w(x))
-  // Element e of lane lo holds ky = lo + TLR*e: elements below E/2 lie in
-  // [0, H), those above E/2 in (H, NY), and only lane 0's elements 0 and E/2
-  // are the real-valued ky = 0 and ky = H, so the mirror and edge tests are
-  // fixed per element once the loop is unrolled.
-  auto build = [&](double2* z, int which, int x, int lo) {
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const int ky = lo + TLR * e;
-      const bool edge = (e == 0 || e == E / 2) && lo == 0;
-      const bool mirror = e > E / 2 || (e == E / 2 && lo != 0);
-      const int kk = mirror ? NY - ky : ky;
-      // a column past the band takes column 0's address and then zero
-      const bool in = !BAND || kk < a.nyc;
-      const int kl = in ? kk : 0;
-      double2 A, B;
-      const double fk = (double)kk;
-      if (which == 0) {         // u = i ky G1, v = G2
-        const double2 g1 = at(a.g[0], gidx(x, kl, ld));
-        A = make_double2(-fk * g1.y, fk * g1.x);
-        B = at(a.g[1], gidx(x, kl, ld));
-      } else if (which == 1) {  // w_x = G3, w_y = i ky G4
-        A = at(a.g[2], gidx(x, kl, ld));
-        const double2 g4 = at(a.g[3], gidx(x, kl, ld));
-        B = make_double2(-fk * g4.y, fk * g4.x);
-      } else if (which == 2) {  // w of rows x and x+1 = G4
-        A = at(a.g[3], gidx(x, kl, ld));
-        B = at(a.g[3], gidx(x + 1, kl, ld));
-      } else {                  // w of row x alone
-        A = at(a.g[3], gidx(x, kl, ld));
-        B = make_double2(0.0, 0.0);
-      }
-      if (edge) { A.y = 0.0; B.y = 0.0; }
-      z[e] = mirror ? make_double2(A.x + B.y, B.x - A.y) : make_double2(A.x - B.y, A.y + B.x);
-      if (!in) z[e] = make_double2(0.0, 0.0);
-      if ((e & 3) == 3) asm volatile("" ::: "memory");
-    }
-  };
+  auto build = [&](double2 (&z)[E], int which, int x, int lo) { rpass_build<NY, TLR, BAND>(z, which, x, lo, a); };
 
   // RP_CFL: this thread's largest pi (|u|/dx + |v|/dy) over its points of
   // u + iv (z1 after its transform); a NaN propagates
@@ -928,28 +933,149 @@ __device__ __forceinline__ void rpass_body_tw(const RPassArgs& a, const int blk,
   }
 }
 
+constexpr int rpass_teams(int PFR) { return (PFR & 7) >= 6 ? 2 : 1; }
+
+// PFR = 6 and 7: a single row on two teams of TLR threads.  Team 0 transforms
+// u + iv, team 1 w_x + i w_y, which it passes to team 0 through LDS; team 0
+// forms the product and transforms it forward (PFR = 7: at half length), while
+// team 1 transforms w where max|w| is wanted.  Two transforms follow one another
+// instead of three (four with max|w|) and each thread loads two fields instead
+// of four.  Bound by that chain while a launch is one round of rows.  us per
+// step against one team: 1024^2 RK4CN 162.9 / 165.2, 512^2 72.4 / 75.5 (CN-AB4,
+// max|w| in every step, 23.7 / 25.2), 256^2 45.4 / 46.4, 128^2 36.2 / 37.8, 64^2 33.9 /
+// 35.5; PFR = 7 ties (1024^2 163.5 and, band-limited, 154.2 against 155.1; 512^2 74.3).
+template <int NY, int TLR, bool HALF, bool CFL, bool BAND, typename TW, typename TWH>
+__device__ __forceinline__ void rpass_team_body(const RPassArgs& a, const int x0, const TW& tw, const TWH& twh) {
+  static_assert(TLR <= 64, "a team fits a wave");
+  constexpr int E = NY / TLR;
+  constexpr int LS = padx_s<RPS>(NY) + 1;
+  __shared__ double2 lds[2 * LS];
+  const int tid = (int)threadIdx.x, team = tid / TLR, l = tid % TLR;
+  const int ld = a.ld;
+  double2* const buf = lds + team * LS;
+  // the wave's maximum (bits of a non-negative double; a NaN compares largest)
+  auto team_max = [&](double m) -> unsigned long long {
+    unsigned long long mb = (unsigned long long)__double_as_longlong(m != m ? __longlong_as_double(0x7ff8000000000000ll) : m);
+#pragma unroll
+    for (int off = TLR / 2; off > 0; off >>= 1) {
+      const unsigned long long o = __shfl_xor(mb, off, 64);
+      mb = o > mb ? o : mb;
+    }
+    return mb;
+  };
+
+  if (a.mode & RP_NL) {
+    double2 z[E];
+    if constexpr (TLR == 64) {   // a team is a wave: one of two uniform branches
+      if (team == 0) rpass_build<NY, TLR, BAND>(z, 0, x0, opaque(l), a);
+      else rpass_build<NY, TLR, BAND>(z, 1, x0, opaque(l), a);
+    } else {
+      const double2* const fa = pick(team != 0, a.g[2], a.g[0]);   // G1, w_x = G3
+      const double2* const fb = pick(team != 0, a.g[3], a.g[1]);   // v = G2, G4
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int ky = l + TLR * e;
+        const bool edge = (e == 0 || e == E / 2) && l == 0;
+        const bool mirror = e > E / 2 || (e == E / 2 && l != 0);
+        const int kk = mirror ? NY - ky : ky;
+        const bool in = !BAND || kk < a.nyc;
+        const size_t idx = gidx(x0, in ? kk : 0, ld);
+        const double2 ga = at(fa, idx), gb = at(fb, idx);
+        const double fk = (double)kk;
+        double2 A = team ? ga : make_double2(-fk * ga.y, fk * ga.x);
+        double2 B = team ? make_double2(-fk * gb.y, fk * gb.x) : gb;
+        if (edge) { A.y = 0.0; B.y = 0.0; }
+        z[e] = mirror ? make_double2(A.x + B.y, B.x - A.y) : make_double2(A.x - B.y, A.y + B.x);
+        if (!in) z[e] = make_double2(0.0, 0.0);
+      }
+    }
+    fft_reg<NY, TLR, +1, false, RPS>(z, buf, tw, opaque(l));
+    if (CFL && (a.mode & RP_CFL)) {
+      double cm = 0.0;
+      if (team == 0) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          const double uu = z[e].x * a.cfl_s, vv = z[e].y * a.cfl_s;
+          const double c = M_PI * (fabs(uu) / a.cfl_dx + fabs(vv) / a.cfl_dy);
+          cm = (c > cm || c != c) ? c : cm;
+        }
+      }
+      const unsigned long long mb = team_max(cm);
+      if (tid == 0) atomicMax(a.cmax, mb);
+    }
+    if (team == 1) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) buf[l + TLR * e] = z[e];
+    }
+    __syncthreads();
+    double2 w[E];
+    if (team == 0) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const double2 o = lds[LS + l + TLR * e];
+        w[e] = make_double2(z[e].x * o.x + z[e].y * o.y, 0.0);   // u*w_x + v*w_y
+      }
+    }
+    __syncthreads();
+    if (team == 0) {
+      if constexpr (HALF) {
+        rpass_forward_half<NY, TLR, false, BAND>(w, buf, a, x0, l, twh);
+      } else {
+        fft_reg<NY, TLR, -1, false, RPS>(w, buf, tw, opaque(l));
+#pragma unroll
+        for (int e = 0; e <= E / 2; ++e) {
+          const int k = l + TLR * e;
+          if (BAND && k >= a.nyc) continue;
+          if (e < E / 2) at(a.nout, nidx(x0, k, ld)) = (e == 0 && l == 0) ? make_double2(w[e].x, 0.0) : w[e];
+          else if (l == 0) at(a.nout, nidx(x0, k, ld)) = make_double2(w[e].x, 0.0);
+        }
+      }
+    }
+  }
+  if ((a.mode & RP_W) && team == 1) {
+    double2 z[E];
+    rpass_build<NY, TLR, BAND>(z, 3, x0, opaque(l), a);
+    fft_reg<NY, TLR, +1, false, RPS>(z, buf, tw, opaque(l));
+    double m = 0.0;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const double w0 = z[e].x * a.wscale;
+      if (a.wreal) at(a.wreal, (size_t)x0 * NY + l + TLR * e) = w0;
+      const double aw = fabs(w0);
+      m = (aw > m || aw != aw) ? aw : m;
+    }
+    const unsigned long long mb = team_max(m);
+    if (l == 0) atomicMax(a.wmax, mb);
+  }
+}
+
 template <int NY, int TLR, int PAIRS, int PFR, bool CFL, bool BAND>
 __device__ __forceinline__ void rpass_body(const RPassArgs& a, const int blk) {
   constexpr int PM = PFR & 7, PX = PFR & 23;
   const int l = (int)threadIdx.x % TLR;
+  auto run = [&](const auto& tw, const auto& twh) {
+    if constexpr (PM >= 6) rpass_team_body<NY, TLR, PM == 7, CFL, BAND>(a, blk, tw, twh);
+    else rpass_body_tw<NY, TLR, PAIRS, PX, CFL, BAND>(a, blk, tw, twh);
+  };
+  constexpr bool HLF = PM == 4 || PM == 5 || PM == 7;
   if constexpr ((PFR & 8) != 0) {
     static_assert(PAIRS == 1 && TLR <= 64, "preloaded twiddle powers are for one-wave rows");
     TwFull<NY, TLR> tw;
     load_twiddles<NY, TLR>(tw, a.tw, l);
-    if constexpr (PM >= 4) {
+    if constexpr (HLF) {
       TwFull<NY / 2, TLR> twh;
       load_twiddles<NY / 2, TLR>(twh, a.tw, half_lane<TLR>(l));
-      rpass_body_tw<NY, TLR, PAIRS, PX, CFL, BAND>(a, blk, tw, twh);
+      run(tw, twh);
     } else {
-      rpass_body_tw<NY, TLR, PAIRS, PX, CFL, BAND>(a, blk, tw, a.tw);
+      run(tw, a.tw);
     }
   } else {
     NS2D_TWIDDLES(NY, TLR, tw, a.tw, l)
-    if constexpr (PM >= 4) {
+    if constexpr (HLF) {
       NS2D_TWIDDLES(NY / 2, TLR, twh, a.tw, half_lane<TLR>(l))
-      rpass_body_tw<NY, TLR, PAIRS, PX, CFL, BAND>(a, blk, tw, twh);
+      run(tw, twh);
     } else {
-      rpass_body_tw<NY, TLR, PAIRS, PX, CFL, BAND>(a, blk, tw, a.tw);
+      run(tw, a.tw);
     }
   }
 }
@@ -1022,18 +1148,18 @@ __device__ __forceinline__ void rpass_forward_half(double2 (&w)[NY / TLR], doubl
 // Consecutive rows (row pairs) go to one XCD, whose L2 then serves the
 // x-tiles of the mixed-space fields that neighbouring rows share.
 template <int NY, int TLR, int PAIRS, int W, int PFR, bool BAND = false>
-__global__ __launch_bounds__(TLR * PAIRS, W) void rpass_kernel(RPassArgs a) {
+__global__ __launch_bounds__(TLR * PAIRS * rpass_teams(PFR), W) void rpass_kernel(RPassArgs a) {
   rpass_body<NY, TLR, PAIRS, PFR, false, BAND>(a, xcd_remap((int)blockIdx.x, (int)gridDim.x));
 }
 
 // the same shape with the CFL-rate reduction compiled in (ns2d_cfl_rate)
 template <int NY, int TLR, int PAIRS, int W, int PFR, bool BAND = false>
-__global__ __launch_bounds__(TLR * PAIRS, W) void rpass_cfl_kernel(RPassArgs a) {
+__global__ __launch_bounds__(TLR * PAIRS * rpass_teams(PFR), W) void rpass_cfl_kernel(RPassArgs a) {
   rpass_body<NY, TLR, PAIRS, PFR, true, BAND>(a, xcd_remap((int)blockIdx.x, (int)gridDim.x));
 }
 
 template <int NY, int TLR, int PAIRS, int W, int PFR, bool BAND = false>
-__global__ __launch_bounds__(TLR * PAIRS, W) void rpass_batched(const RPassArgs* __restrict__ tab, int per_member) {
+__global__ __launch_bounds__(TLR * PAIRS * rpass_teams(PFR), W) void rpass_batched(const RPassArgs* __restrict__ tab, int per_member) {
   const int b = xcd_remap((int)blockIdx.x, (int)gridDim.x);
   const int m = b / per_member;
   rpass_body<NY, TLR, PAIRS, PFR, false, BAND>(tab[m], b - m * per_member);
@@ -1725,16 +1851,20 @@ struct KVariant {
   X(16, 4, 1, 1, 12) \
   X(32, 4, 16, 1, 0) \
   X(32, 16, 1, 1, 3) \
+  X(32, 16, 1, 1, 6) \
   X(32, 2, 32, 1, 0) \
   X(64, 8, 8, 1, 0) \
   X(64, 16, 1, 1, 3) \
+  X(64, 16, 1, 1, 14) \
   X(64, 4, 16, 1, 0) \
   X(128, 16, 4, 1, 0) \
   X(128, 64, 1, 1, 11) \
+  X(128, 64, 1, 1, 14) \
   X(128, 8, 8, 1, 0) \
   X(128, 32, 2, 1, 0) \
   X(256, 64, 1, 1, 11) \
   X(256, 32, 2, 1, 0) \
+  X(256, 64, 1, 1, 6) \
   X(256, 64, 1, 1, 10) \
   X(256, 64, 1, 1, 2) \
   X(256, 64, 1, 1, 0) \
@@ -1744,6 +1874,7 @@ struct KVariant {
   X(256, 64, 1, 1, 4) \
   X(512, 64, 1, 1, 4) \
   X(512, 64, 4, 1, 0) \
+  X(512, 64, 1, 1, 6) \
   X(512, 64, 1, 1, 0) \
   X(512, 64, 1, 1, 2) \
   X(512, 32, 2, 1, 0) \
@@ -1754,6 +1885,7 @@ struct KVariant {
   X(512, 128, 1, 1, 2) \
   X(512, 64, 1, 1, 3) \
   X(1024, 64, 1, 1, 3) \
+  X(1024, 64, 1, 1, 6) \
   X(1024, 256, 1, 1, 2) \
   X(1024, 256, 1, 1, 0) \
   X(1024, 256, 1, 1, 1) \

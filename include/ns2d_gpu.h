@@ -202,7 +202,8 @@ int ns2d_variant_info(int pass, int n, int idx, int* shape4);
  * table instead of forming them by products (row pass only; bit 1 then means
  * its G fields are loaded up front); bit 6: the exchanges pass real and
  * imaginary parts one after another through half the LDS; bit 7: the exchanges
- * alternate between two line buffers. */
+ * alternate between two line buffers; bit 8: a single row runs on two teams of
+ * the stated threads. */
 int ns2d_variant_extra(int pass, int n, int idx, int* extra4);
 /* The shape a new handle with this integrator (NS2D_INT_*) runs on a square
  * grid of length n (other grids may start from a neighbouring index) unless NS2D_KPASS_VARIANT_<Nx> / NS2D_RPASS_VARIANT_<Ny>
