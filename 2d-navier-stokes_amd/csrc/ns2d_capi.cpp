@@ -84,13 +84,19 @@ struct ns2d_handle {
   PhysArgs ph{};
   // hipGraph of one period of steps (kernel launches only; see step_impl)
   bool use_graph = true;
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t gexec = nullptr;
-  struct {
-    double dt;
-    int wcur, cur, ring, kvar, rvar, check, period, band;
-    const double* lam;
-  } gkey{};
+  // (two of them: a program that takes an odd number of steps per call starts
+  // its periods from either state buffer in turn)
+  struct StepGraph {
+    hipGraphExec_t exec = nullptr;
+    double dt = 0.0;
+    int wcur = 0, cur = 0, ring = 0, kvar = 0, rvar = 0, check = 0, period = 0, band = 0;
+    const double* lam = nullptr;
+    bool same(const StepGraph& o) const {
+      return dt == o.dt && wcur == o.wcur && cur == o.cur && ring == o.ring && kvar == o.kvar && rvar == o.rvar &&
+             check == o.check && period == o.period && band == o.band && lam == o.lam;
+    }
+  } step_graph[2];
+  int step_graph_last = 0;   // the one replayed last
   // adjoint buffers (allocated on first use)
   double2* tape = nullptr;     // the tape in use: [slot][4 fields][M], slot = 4*step + stage
   double2* tape_buf[2] = {nullptr, nullptr};  // second one only when it fits (overlap)
@@ -368,11 +374,9 @@ int read_stat(ns2d_handle* h, unsigned long long* st) {
   return NS2D_OK;
 }
 
-int reset_stat(ns2d_handle* h) {
-  unsigned long long st[STAT_SPILL] = {0ull, 0ull, ~0ull, 0ull, 0ull};
-  HIPCHK(hipMemcpyAsync(h->stat, st, sizeof st, hipMemcpyHostToDevice, h->stream));
-  HIPCHK(hipStreamSynchronize(h->stream));
-  return NS2D_OK;
+int stat_op(ns2d_handle* h, int op) {
+  const hipError_t e = launch_stat(h->stat, op, h->stream);
+  return e == hipSuccess ? NS2D_OK : fail(NS2D_ERR_HIP, "status launch: %s", hipGetErrorString(e));
 }
 
 // max|w| of the state into stat[WMAX_CUR] (after clearing it)
@@ -380,8 +384,8 @@ int state_wmax(ns2d_handle* h, double* out, double* wreal) {
   h->band_on = band_now(h);
   int rc = prepare_inv(h);
   if (rc) return rc;
-  const unsigned long long zero = 0ull;
-  HIPCHK(hipMemcpyAsync(h->stat + STAT_WMAX_CUR, &zero, sizeof zero, hipMemcpyHostToDevice, h->stream));
+  rc = stat_op(h, STAT_OP_CLEAR_WMAX);
+  if (rc) return rc;
   RPassArgs a = rbase(h, RP_W);
   a.wreal = wreal;
   rc = run_rpass(h, a);
@@ -401,8 +405,8 @@ int state_cfl(ns2d_handle* h, double* out) {
   h->band_on = band_now(h);
   int rc = prepare_inv(h);
   if (rc) return rc;
-  const unsigned long long zero = 0ull;
-  HIPCHK(hipMemcpyAsync(h->stat + STAT_CFL, &zero, sizeof zero, hipMemcpyHostToDevice, h->stream));
+  rc = stat_op(h, STAT_OP_CLEAR_CFL);
+  if (rc) return rc;
   RPassArgs a = rbase(h, RP_NL | RP_CFL);
   a.cmax = h->stat + STAT_CFL;
   a.cfl_s = 1.0 / (double)((long)h->p.nx * h->p.ny);
@@ -668,13 +672,14 @@ static int create_impl(const ns2d_params* p, hipStream_t ext_stream, ns2d_t** ou
   }
   if (hipMemsetAsync(h->stat, 0, sizeof(unsigned long long) * STAT_N, h->stream) != hipSuccess)
     return cleanup(fail(NS2D_ERR_HIP, "memset failed"));
-  int rc = reset_stat(h);
+  int rc = stat_op(h, STAT_OP_RESET);
+  if (rc == NS2D_OK && hipStreamSynchronize(h->stream) != hipSuccess) rc = fail(NS2D_ERR_HIP, "stream synchronize failed");
   if (rc) return cleanup(rc);
   *out = h;
   return NS2D_OK;
 }
 
-static void drop_graph(ns2d_handle* h);
+static void drop_graph(ns2d_handle* h, ns2d_handle::StepGraph& g);
 
 int ns2d_destroy(ns2d_t* h) {
   if (!h) return NS2D_OK;
@@ -697,7 +702,7 @@ int ns2d_destroy(ns2d_t* h) {
   if (h->wreal) (void)hipFree(h->wreal);
   if (h->rbuf) (void)hipFree(h->rbuf);
   if (h->stage) (void)hipFree(h->stage);
-  drop_graph(h);
+  for (auto& g : h->step_graph) drop_graph(h, g);
   for (auto& g : h->adj_graph)
     if (g.exec) (void)hipGraphExecDestroy(g.exec);
   if (h->ev_fork) (void)hipEventDestroy(h->ev_fork);
@@ -734,11 +739,13 @@ static int load_state(ns2d_t* h, const void* src, hipMemcpyKind kind) {
 static int set_state_impl(ns2d_t* h, const void* src, hipMemcpyKind kind) {
   if (!h || !src) return fail(NS2D_ERR_INVALID, "null argument");
   HIPCHK(hipSetDevice(h->p.device));
-  int rc0 = load_state(h, src, kind);
+  int rc0 = stat_op(h, STAT_OP_RESET);
+  if (rc0 == NS2D_OK) rc0 = load_state(h, src, kind);
   if (rc0) return rc0;
   h->iters = 0;
   h->hyper_eff = h->p.hyper_flag;
-  return reset_stat(h);
+  if (h->kc == 0) HIPCHK(hipStreamSynchronize(h->stream));   // (load_state has waited otherwise)
+  return NS2D_OK;
 }
 
 static int get_state_impl(ns2d_t* h, void* dst, hipMemcpyKind kind) {
@@ -755,12 +762,11 @@ int ns2d_get_state(ns2d_t* h, double* w_hat) { return get_state_impl(h, w_hat, h
 int ns2d_set_state_device(ns2d_t* h, const void* d) { return set_state_impl(h, d, hipMemcpyDeviceToDevice); }
 int ns2d_get_state_device(ns2d_t* h, void* d) { return get_state_impl(h, d, hipMemcpyDeviceToDevice); }
 
-static void drop_graph(ns2d_handle* h) {
-  if (h->gexec && h->stream) (void)hipStreamSynchronize(h->stream);   // a replay may still be running
-  if (h->gexec) (void)hipGraphExecDestroy(h->gexec);
-  if (h->graph) (void)hipGraphDestroy(h->graph);
-  h->gexec = nullptr;
-  h->graph = nullptr;
+static void drop_graph(ns2d_handle* h, ns2d_handle::StepGraph& g) {
+  if (!g.exec) return;
+  if (h->stream) (void)hipStreamSynchronize(h->stream);   // a replay may still be running
+  (void)hipGraphExecDestroy(g.exec);
+  g.exec = nullptr;
 }
 
 // One direct step of the configured integrator.
@@ -775,13 +781,23 @@ static int one_step(ns2d_handle* h, double dt, bool check) {
 static int graph_steps(ns2d_handle* h, double dt, bool check, int period) {
   const double* lam = lam_table(h, h->p.integrator == NS2D_INT_AB4 ? visc_kind_plain(h) : visc_kind_rk(h));
   if (!lam) return fail(NS2D_ERR_HIP, "coefficient table allocation failed");
-  const int ring = h->p.integrator == NS2D_INT_AB4 ? (int)((h->iters + 1 - 4) % 4) : 0;
-  const bool same = h->gexec && h->gkey.dt == dt && h->gkey.wcur == h->wcur && h->gkey.cur == h->cur &&
-                    h->gkey.ring == ring && h->gkey.kvar == h->kvar && h->gkey.rvar == h->rvar &&
-                    h->gkey.check == (int)check && h->gkey.period == period && h->gkey.lam == lam &&
-                    h->gkey.band == (int)h->band_on;
-  if (!same) {
-    drop_graph(h);
+  ns2d_handle::StepGraph key;
+  key.dt = dt;
+  key.wcur = h->wcur;
+  key.cur = h->cur;
+  key.ring = h->p.integrator == NS2D_INT_AB4 ? (int)((h->iters + 1 - 4) % 4) : 0;
+  key.kvar = h->kvar;
+  key.rvar = h->rvar;
+  key.check = check;
+  key.period = period;
+  key.band = h->band_on;
+  key.lam = lam;
+  int slot = -1;
+  for (int i = 0; i < 2; ++i)
+    if (h->step_graph[i].exec && h->step_graph[i].same(key)) slot = i;
+  if (slot < 0) {
+    slot = !h->step_graph[0].exec ? 0 : !h->step_graph[1].exec ? 1 : 1 - h->step_graph_last;
+    drop_graph(h, h->step_graph[slot]);
     const int cur0 = h->cur, wcur0 = h->wcur, hyp0 = h->hyper_eff;
     const long it0 = h->iters;
     HIPCHK(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
@@ -798,20 +814,13 @@ static int graph_steps(ns2d_handle* h, double dt, bool check, int period) {
       return rc;
     }
     if (ec != hipSuccess) return fail(NS2D_ERR_HIP, "graph capture: %s", hipGetErrorString(ec));
-    h->graph = g;
-    HIPCHK(hipGraphInstantiate(&h->gexec, g, nullptr, nullptr, 0));
-    h->gkey.dt = dt;
-    h->gkey.wcur = h->wcur;
-    h->gkey.cur = h->cur;
-    h->gkey.ring = ring;
-    h->gkey.kvar = h->kvar;
-    h->gkey.rvar = h->rvar;
-    h->gkey.check = check;
-    h->gkey.period = period;
-    h->gkey.lam = lam;
-    h->gkey.band = h->band_on;
+    const hipError_t ei = hipGraphInstantiate(&key.exec, g, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(g);
+    if (ei != hipSuccess) return fail(NS2D_ERR_HIP, "graph instantiate: %s", hipGetErrorString(ei));
+    h->step_graph[slot] = key;
   }
-  HIPCHK(hipGraphLaunch(h->gexec, h->stream));
+  h->step_graph_last = slot;
+  HIPCHK(hipGraphLaunch(h->step_graph[slot].exec, h->stream));
   h->iters += period;  // cur and wcur are back to their values after a period
   return NS2D_OK;
 }
@@ -853,16 +862,11 @@ static int step_impl(ns2d_t* h, double dt, long nsteps) {
     hipError_t e = launch_rpass(h->p.nx, h->p.ny, h->rvar, a, h->stream);
     ev_end(h);
     if (e != hipSuccess) return fail(NS2D_ERR_HIP, "rpass launch: %s", hipGetErrorString(e));
+    rc = stat_op(h, STAT_OP_CHECK);
+    if (rc) return rc;
     unsigned long long st[STAT_N];
     rc = read_stat(h, st);
     if (rc) return rc;
-    double m;
-    std::memcpy(&m, &st[STAT_WMAX_CUR], sizeof m);
-    if (!(m < MAX_VORT_LIM) && st[STAT_FIRST_BAD] == ~0ull) st[STAT_FIRST_BAD] = st[STAT_ITER];
-    st[STAT_WMAX_LAST] = st[STAT_WMAX_CUR];
-    st[STAT_WMAX_CUR] = 0ull;
-    HIPCHK(hipMemcpyAsync(h->stat, st, sizeof st, hipMemcpyHostToDevice, h->stream));
-    HIPCHK(hipStreamSynchronize(h->stream));
     if (st[STAT_FIRST_BAD] != ~0ull)
       return fail(NS2D_ERR_BLOWUP, "System has reached maximum Vorticity limit at Iter: [%llu]",
                   (unsigned long long)st[STAT_FIRST_BAD]);
@@ -1115,8 +1119,8 @@ int ns2d_c2r(ns2d_t* h, const double* w_hat, double* w) {
   rc = run_rpass(h, r);
   if (rc) return rc;
   // the row pass also folded max|w| into the step check's accumulator
-  const unsigned long long zero = 0ull;
-  HIPCHK(hipMemcpyAsync(h->stat + STAT_WMAX_CUR, &zero, sizeof zero, hipMemcpyHostToDevice, h->stream));
+  rc = stat_op(h, STAT_OP_CLEAR_WMAX);
+  if (rc) return rc;
   HIPCHK(hipMemcpyAsync(w, h->wreal, sizeof(double) * n, hipMemcpyDeviceToHost, h->stream));
   HIPCHK(hipStreamSynchronize(h->stream));
   return NS2D_OK;
@@ -1217,6 +1221,9 @@ struct ns2d_ensemble {
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   int graph_parity = -1;
+  // the members' status words and the first member whose check failed (-1: none)
+  unsigned long long** stats = nullptr;
+  int* bad = nullptr;
 };
 
 namespace {
@@ -1665,20 +1672,17 @@ int ns2d_ens_step(ns2d_ens_t* e, const double* dt, long nsteps) {
       hipError_t r = launch_rpass(h->p.nx, h->p.ny, h->rvar, a, e->stream);
       if (r != hipSuccess) return fail(NS2D_ERR_HIP, "rpass launch: %s", hipGetErrorString(r));
     }
-    int bad = -1;
-    for (size_t i = 0; i < e->m.size(); ++i) {
-      ns2d_handle* h = e->m[i];
-      unsigned long long st[STAT_N];
-      int rc = read_stat(h, st);
-      if (rc) return rc;
-      double mx;
-      std::memcpy(&mx, &st[STAT_WMAX_CUR], sizeof mx);
-      if (!(mx < MAX_VORT_LIM) && st[STAT_FIRST_BAD] == ~0ull) st[STAT_FIRST_BAD] = st[STAT_ITER];
-      st[STAT_WMAX_LAST] = st[STAT_WMAX_CUR];
-      st[STAT_WMAX_CUR] = 0ull;
-      HIPCHK(hipMemcpyAsync(h->stat, st, sizeof st, hipMemcpyHostToDevice, e->stream));
-      if (st[STAT_FIRST_BAD] != ~0ull && bad < 0) bad = (int)i;
+    const int nm = (int)e->m.size();
+    if (!e->stats) {
+      std::vector<unsigned long long*> p(nm);
+      for (int i = 0; i < nm; ++i) p[i] = e->m[i]->stat;
+      HIPCHK(hipMalloc((void**)&e->stats, sizeof(unsigned long long*) * nm));
+      HIPCHK(upload(e->stream, e->stats, p.data(), sizeof(unsigned long long*) * nm));
     }
+    if (!e->bad) HIPCHK(hipMalloc((void**)&e->bad, sizeof(int)));
+    HIPCHK(launch_stat_check_all(e->stats, nm, e->bad, e->stream));
+    int bad = -1;
+    HIPCHK(hipMemcpyAsync(&bad, e->bad, sizeof bad, hipMemcpyDeviceToHost, e->stream));
     HIPCHK(hipStreamSynchronize(e->stream));
     if (bad >= 0) return fail(NS2D_ERR_BLOWUP, "ensemble member %d reached the maximum vorticity limit", bad);
   }
@@ -1727,6 +1731,8 @@ int ns2d_ens_destroy(ns2d_ens_t* e) {
     if (c.done) (void)hipEventDestroy(c.done);
     if (c.stream) (void)hipStreamDestroy(c.stream);
   }
+  if (e->stats) (void)hipFree(e->stats);
+  if (e->bad) (void)hipFree(e->bad);
   for (ns2d_handle* h : e->m) ns2d_destroy(h);
   if (e->fork) (void)hipEventDestroy(e->fork);
   if (e->stream) (void)hipStreamDestroy(e->stream);

@@ -228,16 +228,18 @@ int kpass_variant_extra(int nx, int idx, int* W, int* PS, int* OFF, int* PK);
 unsigned long long shape_table_hash(int nx, int ny);
 hipError_t launch_r2c_rows(int nx, int ny, const double* in, double2* out, const double2* tw, int ld,
                            hipStream_t s);
+// operations on a handle's status words (one thread): the words of a new state;
+// the final step's SystemCheck (solver.c:2301-2326) with the maximum reset; a
+// single word cleared
+enum { STAT_OP_RESET = 0, STAT_OP_CHECK = 1, STAT_OP_CLEAR_WMAX = 2, STAT_OP_CLEAR_CFL = 3 };
+hipError_t launch_stat(unsigned long long* stat, int op, hipStream_t s);
+// STAT_OP_CHECK on n handles' words; *bad: the first one with a failed check, or -1
+hipError_t launch_stat_check_all(unsigned long long* const* stats, int n, int* bad, hipStream_t s);
 hipError_t launch_measures(int nbins, const MeasArgs& a, hipStream_t s);
 // dir 0 (into the device layout), kc2 > 0: *spill = epoch when a mode with
 // |k|^2 >= kc2 is not zero.  dir 1, kc2 > 0: those modes are taken as zero.
 hipError_t launch_relayout(const double2* src, double2* dst, int nx, int nyf, int ld, int dir, long kc2,
                            unsigned long long* spill, unsigned long long epoch, hipStream_t s);
-hipError_t launch_measures(int nbins, const MeasArgs& a, hipStream_t s);
-// dir 0 (into the device layout) with kc2 > 0: *spill (device) becomes
-// nonzero when a mode with |k|^2 >= kc2 is not zero
-hipError_t launch_relayout(const double2* src, double2* dst, int nx, int nyf, int ld, int dir, long kc2,
-                           unsigned long long* spill, hipStream_t s);
 
 // allocation-free measures: per-device scratch (ns2d_noalloc.hip) sized for
 // the spectrum length of a 4096 x 4096 grid (sys_msr.c:394)
