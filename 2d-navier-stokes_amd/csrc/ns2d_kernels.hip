@@ -186,7 +186,7 @@ int kpass_variant_extra(int nx, int idx, int* W, int* PS, int* OFF, int* PK) {
   *PS = v->PS;
   *OFF = v->OFF;
   *PK = (v->PK != 0) | ((v->PF & 1) << 1) | ((v->PK == 2) << 2) | (((v->PF & 2) != 0) << 6) |
-        (((v->PF & 4) != 0) << 7);
+        (((v->PF & 4) != 0) << 7) | (((v->PF & 8) != 0) << 5);
   return 0;
 }
 

@@ -167,8 +167,8 @@ __device__ __forceinline__ double dealias_factor(const PhysArgs& ph, int kx, int
 // 4096^2 CN-AB4 16.28 -> 10.84 ms per 15 steps, 512^2 RK4CN 2.76 -> 2.46 ms
 // per 30, a 24-member ensemble 14.8 -> 12.2 ms per 12; 256^2 and below, where a
 // pass is one chain of latencies, do not change.
-template <int L, int C, int T, int KS, int PS, int OFF, int PK, int PFX, bool BAND>
-__device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
+template <int L, int C, int T, int KS, int PS, int OFF, int PK, int PFX, bool BAND, typename TW>
+__device__ __forceinline__ void kpass_body_tw(const KPassArgs& a, const int wi, const TW& tw) {
   constexpr int PF = PFX & 1;
   constexpr bool SPL = (PFX & 2) != 0;   // exchanges of doubles (fft_reg)
   constexpr bool DBL = (PFX & 4) != 0;   // exchanges alternate between two buffers (fft_reg)
@@ -215,7 +215,6 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
   const bool writer = split == 0;
   const PhysArgs& ph = a.ph;
   double2* buf = reinterpret_cast<double2*>(lds + c * LS * (SPL ? 1 : 2));
-  NS2D_TWIDDLES(L, TL, tw, a.tw, l)
   // the pair's held columns (see above)
   double2* __restrict__ hold = a.pairbuf + (size_t)split * 2 * L;
 
@@ -608,6 +607,22 @@ __device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
 #pragma unroll
       for (int e = 0; e < E; ++e) at(gout, gidx(l_o + TL * e, ky_o, ld)) = F[e];
     }
+  }
+}
+
+// PFX & 8: every twiddle power of the shape's transforms preloaded (TwFull)
+// instead of one load per butterfly inside each pass.
+template <int L, int C, int T, int KS, int PS, int OFF, int PK, int PFX, bool BAND>
+__device__ __forceinline__ void kpass_body(const KPassArgs& a, const int wi) {
+  constexpr int TL = T / C;
+  const int l = (int)threadIdx.x / C;
+  if constexpr ((PFX & 8) != 0) {
+    TwFull<L, TL> tw;
+    load_twiddles<L, TL>(tw, a.tw, l);
+    kpass_body_tw<L, C, T, KS, PS, OFF, PK, PFX, BAND>(a, wi, tw);
+  } else {
+    NS2D_TWIDDLES(L, TL, tw, a.tw, l)
+    kpass_body_tw<L, C, T, KS, PS, OFF, PK, PFX, BAND>(a, wi, tw);
   }
 }
 
@@ -1660,7 +1675,10 @@ __global__ __launch_bounds__(T) void measures_kernel(MeasArgs a) {
 // two line buffers (one barrier each instead of two) where the grid leaves the
 // LDS: 512 points 15.7 -> 15.1 us per launch (257 columns), 13.4 -> 13.0 (171);
 // 1024 points 23.6 -> 22.6 (341 columns), but 24.3 -> 28.1 at 513, whose 1026
-// workgroups need a fifth on two CUs.
+// workgroups need a fifth on two CUs.  PF = 8 preloads the twiddle powers: up to
+// 256 points, where the loads inside the passes lengthen the chain, 64^2 33.8 -> 32.0 us
+// per step, 128^2 36.1 -> 33.5, 256^2 45.1 -> 44.0; at 512 and 1024 the registers cost
+// more (512^2 71.7 -> 73.5, 1024^2 162.7 -> 178.9).
 #define NS2D_KPASS_VARIANTS(X) \
   X(8, 16, 64, 4, 3, 1, 0, 1, 0) \
   X(8, 16, 64, 1, 3, 1, 0, 1, 0) \
@@ -1668,18 +1686,19 @@ __global__ __launch_bounds__(T) void measures_kernel(MeasArgs a) {
   X(16, 8, 64, 4, 3, 1, 0, 1, 0) \
   X(16, 16, 64, 1, 3, 1, 0, 1, 0) \
   X(16, 16, 64, 1, 3, 1, 1, 1, 0) \
-  X(32, 4, 64, 4, 3, 1, 0, 1, 0) \
+  X(32, 4, 64, 4, 3, 1, 0, 1, 8) \
   X(32, 16, 64, 1, 3, 1, 0, 1, 0) \
   X(32, 16, 64, 1, 3, 1, 1, 1, 0) \
-  X(64, 2, 64, 4, 3, 1, 0, 1, 0) \
+  X(64, 2, 64, 4, 3, 1, 0, 1, 8) \
   X(64, 16, 64, 1, 3, 1, 0, 1, 0) \
   X(64, 16, 64, 1, 3, 1, 1, 1, 0) \
-  X(128, 1, 64, 4, 3, 1, 0, 1, 0) \
+  X(128, 1, 64, 4, 3, 1, 0, 1, 8) \
   X(128, 2, 64, 4, 3, 1, 0, 1, 0) \
   X(128, 16, 128, 1, 3, 1, 0, 1, 0) \
   X(128, 16, 128, 1, 3, 1, 1, 1, 0) \
   X(128, 8, 64, 2, 3, 1, 1, 1, 0) \
   X(128, 8, 128, 2, 3, 1, 1, 1, 0) \
+  X(256, 1, 64, 4, 3, 1, 0, 1, 8) \
   X(256, 1, 64, 4, 3, 1, 0, 1, 0) \
   X(256, 1, 64, 4, 3, 1, 0, 1, 1) \
   X(256, 8, 512, 2, 3, 1, 0, 1, 0) \

@@ -198,8 +198,8 @@ int ns2d_variant_info(int pass, int n, int idx, int* shape4);
  * bit 2: the packed pair's second column stays in registers; bit 3: the row
  * pass runs one row per line group instead of a row pair; bit 4: that row's
  * real product is transformed forward as a complex line of half the length;
- * bit 5: the row transforms multiply by twiddle powers preloaded from the
- * table instead of forming them by products (row pass only; bit 1 then means
+ * bit 5: the transforms multiply by twiddle powers preloaded from the table
+ * instead of forming them by products (in the row pass bit 1 then means that
  * its G fields are loaded up front); bit 6: the exchanges pass real and
  * imaginary parts one after another through half the LDS; bit 7: the exchanges
  * alternate between two line buffers; bit 8: a single row runs on two teams of
