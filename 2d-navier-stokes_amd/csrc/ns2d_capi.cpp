@@ -821,6 +821,7 @@ static int graph_steps(ns2d_handle* h, double dt, bool check, int period) {
   }
   h->step_graph_last = slot;
   HIPCHK(hipGraphLaunch(h->step_graph[slot].exec, h->stream));
+  if (h->p.integrator != NS2D_INT_AB4) after_rk_update(h);
   h->iters += period;  // cur and wcur are back to their values after a period
   return NS2D_OK;
 }
@@ -841,9 +842,10 @@ static int step_impl(ns2d_t* h, double dt, long nsteps) {
   long s = 0;
   while (s < nsteps) {
     // graphs only once the integrator's arguments are periodic: after the AB4
-    // start-up and after the viscous-flag update of the first RK4CN step
-    const bool settled = !(ab4 && h->iters < 3) &&
-                         !((h->p.quirks & NS2D_QUIRK_VISC_ASSIGN) && h->p.drag_flag != 1 && h->hyper_eff != 1);
+    // start-up (the viscous-flag update of the first RK4CN step does not change
+    // RK4CN's coefficients, visc_kind_rk: where the flag is assigned they are
+    // VISC_HYPER's before and after)
+    const bool settled = !(ab4 && h->iters < 3);
     if (h->use_graph && !h->profiling && settled && nsteps - s >= period) {
       rc = graph_steps(h, dt, check, period);
       s += period;
@@ -1597,19 +1599,6 @@ int ns2d_ens_step(ns2d_ens_t* e, const double* dt, long nsteps) {
     if (h->wcur != e->m[0]->wcur) return fail(NS2D_ERR_STATE, "ensemble members out of step");
   }
   long s = 0;
-  // first steps one member at a time until the viscous flags have settled (Q3)
-  while (s < nsteps) {
-    bool settled = true;
-    for (ns2d_handle* h : e->m)
-      settled = settled && !((h->p.quirks & NS2D_QUIRK_VISC_ASSIGN) && h->p.drag_flag != 1 && h->hyper_eff != 1);
-    if (settled) break;
-    for (size_t i = 0; i < e->m.size(); ++i) {
-      int rc = rk4cn_step(e->m[i], e->dt[i], check);
-      if (rc) return rc;
-    }
-    e->tables_ok = false;
-    ++s;
-  }
   if (s < nsteps && !e->tuned) {
     // NS2D_ENS_TUNE: 0 keeps the plain solver's shapes, 2 re-tunes ignoring
     // the schedule cache, otherwise a cached schedule for these classes on
