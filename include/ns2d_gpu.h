@@ -181,9 +181,8 @@ int ns2d_profile_steps(ns2d_t* h, double dt, long nsteps, double* kpass_ms, doub
  *                      workgroups sharing a column group}
  *   row pass (Ny):    {threads per row pair, points per thread, threads,
  *                      row pairs per workgroup}
- * The project's autotuner times them and picks one per grid; a new handle
- * starts from ns2d_default_variant's shape (index 0 for both integrators;
- * the integrator argument lets a table name different ones).  No counterpart in the reference (FFTW_MEASURE
+ * A new handle starts from the shape measured fastest for its grid and
+ * integrator.  No counterpart in the reference (FFTW_MEASURE
  * planning, solver.c:2883-2895, plays this role there). */
 #define NS2D_PASS_COLUMN 0
 #define NS2D_PASS_ROW 1
@@ -205,9 +204,10 @@ int ns2d_variant_info(int pass, int n, int idx, int* shape4);
  * alternate between two line buffers; bit 8: a single row runs on two teams of
  * the stated threads. */
 int ns2d_variant_extra(int pass, int n, int idx, int* extra4);
-/* The shape a new handle with this integrator (NS2D_INT_*) runs on a square
- * grid of length n (other grids may start from a neighbouring index) unless NS2D_KPASS_VARIANT_<Nx> / NS2D_RPASS_VARIANT_<Ny>
- * name another.  Needs no GPU. */
+/* The first shape of the table for length n and this integrator (NS2D_INT_*),
+ * index 0.  A new handle starts from the one measured fastest for its rows and
+ * columns together, which can be another index, unless
+ * NS2D_KPASS_VARIANT_<Nx> / NS2D_RPASS_VARIANT_<Ny> name one.  Needs no GPU. */
 int ns2d_default_variant(int pass, int n, int integrator, int* idx);
 int ns2d_set_variant(ns2d_t* h, int pass, int idx);
 /* Device storage of the spectral arrays this library was compiled with:
